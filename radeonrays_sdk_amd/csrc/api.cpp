@@ -1346,11 +1346,11 @@ RRError rrxCmdBuildGeometryBatch(RRContext context, RRBuildOperation build_opera
             b.index16 = m.index16;
             b.tri_count = m.tri_count;
             b.flags = (restructure && m.tri_count >= 64) ? rr::kAccelFlagRestructured : 0u;
-            b.first_chunk = chunks;
-            chunks += rr::RefitChunks(m.tri_count);
+            const uint32_t mesh_chunks = rr::RefitChunks(m.tri_count);
+            b.first_chunk = rr::BatchFirstChunk(chunks, mesh_chunks);
+            chunks = b.first_chunk + mesh_chunks;
             host[k] = b;
         }
-        const uint32_t big_chunks = big < n_small ? host[big].first_chunk : chunks;  // chunks of the big meshes
         const size_t roots_offset = plan.roots_offset;
         const uint32_t max_roots[3] = {plan.max_roots[0], plan.max_roots[1], plan.max_roots[2]};
         auto cmd = [=](hipStream_t s) {
@@ -1361,7 +1361,7 @@ RRError rrxCmdBuildGeometryBatch(RRContext context, RRBuildOperation build_opera
                 if (update) {
                     rr::BatchRefit(table, n_small, chunks, scratch, s);
                 } else {
-                    rr::BatchBuild(table, n_small, big, small, big_chunks, chunks, scratch, s);
+                    rr::BatchBuild(table, n_small, big, small, chunks, scratch, s);
                     // Treelet restructuring of all meshes at once, each in its own work area.
                     if (restructure)
                         rr::BatchRestructure(table, n_small, chunks, max_roots, scratch,

@@ -24,13 +24,13 @@ struct BatchMesh {
     uint32_t index16;
     uint32_t tri_count;
     uint32_t flags;        // header flags of the result (kAccelFlag*)
-    uint32_t first_chunk;  // refit chunks (kRefitChunk leaves) of the meshes before this one
+    uint32_t first_chunk;  // first refit chunk (kRefitChunk leaves), see BatchFirstChunk
     uint32_t pad[2];
 };
 static_assert(sizeof(BatchMesh) == 64, "BatchMesh must be 64 bytes");
 
-// Bytes of a mesh's work area: keys, values and their ping-pong copies, or
-// the treelet-restructuring scratch if that is larger.
+// Bytes of a mesh's work area: keys, values, their ping-pong copies and the
+// tree scratch, or the treelet-restructuring scratch if that is larger.
 size_t BatchWorkBytes(uint32_t tris);
 
 // Scratch head of a batch: queue counter, then the mesh table.
@@ -42,6 +42,14 @@ inline size_t BatchHeadBytes(uint32_t meshes) {
 // Leaves per refit queue entry.
 constexpr uint32_t kRefitChunk = 64;
 inline uint32_t RefitChunks(uint32_t tris) { return (tris + kRefitChunk - 1) / kRefitChunk; }
+// First chunk of a mesh of `chunks` chunks when `before` chunks precede it:
+// meshes do not cross a workgroup of the tree kernel unless they start one.
+constexpr uint32_t kBatchChunksPerWindow = 8;
+inline uint32_t BatchFirstChunk(uint32_t before, uint32_t chunks) {
+    return before % kBatchChunksPerWindow + chunks > kBatchChunksPerWindow
+               ? (before + kBatchChunksPerWindow - 1) / kBatchChunksPerWindow * kBatchChunksPerWindow
+               : before;
+}
 
 // Meshes of at most this many triangles are built with their whole sort in
 // LDS (one 1024-thread workgroup per mesh; 256 threads for meshes of at
@@ -53,16 +61,13 @@ constexpr uint32_t kBatchLdsSmallMaxTris = 4096;
 // `table`, inside `scratch`).  The first `big` meshes (those above
 // kBatchLdsMaxTris triangles; the table is ordered largest first): each
 // workgroup takes the next mesh from a queue and runs bounds, Morton codes
-// and a stable four-pass radix sort through the mesh's work area; then one
-// thread per node of these meshes (in chunks of kRefitChunk leaves, the
-// first big_chunks chunks) emits the hierarchy.  Every other mesh is sorted
-// by one workgroup in LDS, which then emits its hierarchy from the
-// LDS-resident codes; meshes from index `small` on (at most
-// kBatchLdsSmallMaxTris triangles) by 256-thread workgroups.  Last,
-// BatchRefit over all total_chunks chunks.  The results equal BuildBlas
-// with restructure off, mesh by mesh.
-void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t small, uint32_t big_chunks,
-                uint32_t total_chunks, void* scratch, hipStream_t stream);
+// and a stable four-pass radix sort through the mesh's work area.  Every
+// other mesh is sorted by one workgroup in LDS; meshes from index `small` on
+// (at most kBatchLdsSmallMaxTris triangles) by 256-thread workgroups.  Then
+// one launch builds the trees of all total_chunks chunks.  The results equal
+// BuildBlas with restructure off, mesh by mesh.
+void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t small, uint32_t total_chunks,
+                void* scratch, hipStream_t stream);
 
 // Refit of every mesh in the table (the topology of each BLAS is kept), as
 // UpdateBlas mesh by mesh (one launch over the refit chunks of all meshes).

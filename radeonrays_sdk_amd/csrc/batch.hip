@@ -1,15 +1,15 @@
 // batch.hip — batched BLAS build and refit for gfx950.
 //
-// Many small meshes (up to kBatchMaxTris triangles each) are built by three
-// launches.  A persistent one in which each workgroup takes the next mesh
-// from a queue (the host orders the table largest first) and runs the
-// mesh-wide steps of the single-mesh builder with block-level
-// synchronisation only — bounds (wave64 reductions), Morton codes and a
-// stable LSD radix sort of the (code, index) pairs in four 8-bit passes;
-// then Karras emission and the bottom-up refit, one thread per node or leaf
-// of any mesh.  Every step computes exactly what the single-mesh kernels
-// compute (min/max are exact, the sort is stable, emission and refit are the
-// shared device functions), so each result equals BuildBlas of that mesh.
+// Many small meshes (up to kBatchMaxTris triangles each) are built by a few
+// launches: persistent ones in which each workgroup takes the next mesh from
+// a queue (the host orders the table largest first) and runs the mesh-wide
+// steps of the single-mesh builder with block-level synchronisation only —
+// bounds (wave64 reductions), Morton codes and a stable LSD radix sort of the
+// (code, index) pairs in four 8-bit passes; then one that builds the trees of
+// all meshes with their boxes, one thread per leaf of any mesh.  Every step
+// computes exactly what the single-mesh kernels compute (min/max are exact,
+// the sort is stable, the tree is the shared device functions'), so each
+// result equals BuildBlas of that mesh.
 // Behavioural spec of each step: as build.hip (vlk/hlbvh_builder.cpp:159-351).
 #include <hip/hip_runtime.h>
 
@@ -20,6 +20,7 @@
 #include "build_device.h"
 #include "rr_device.h"
 #include "sort.h"
+#include "tree_device.h"
 
 namespace rr {
 
@@ -138,6 +139,20 @@ __device__ void BlockSortPass(const uint32_t* __restrict__ ki, const uint32_t* _
     }
 }
 
+// The tree scratch of a mesh, after its keys, values and their ping-pong
+// copies in the work area.
+__host__ __device__ inline size_t BatchTreeOffset(uint32_t tris) { return AlignUp(tris, 64) * 16; }
+__device__ __forceinline__ void* BatchTreeScratch(uint32_t* work, uint32_t n) {
+    return reinterpret_cast<uint8_t*>(work) + BatchTreeOffset(n);
+}
+__device__ __forceinline__ void ClearTreeCounters(void* tree, uint32_t n, uint32_t tid, uint32_t threads) {
+    const uint32_t windows = TreeWindows(n);
+    if (windows <= 1) return;
+    const uint32_t runs = TreeRuns(windows);
+    const TreeScratch ts = CarveTreeScratch(tree, runs);
+    for (uint32_t i = tid; i < runs; i += threads) ts.arrived[i] = 0;
+}
+
 __global__ void BatchQueueInitKernel(uint32_t* queue) {
     if (threadIdx.x == 0) queue[0] = 0;
     if (threadIdx.x == kBatchLdsQueueWord) queue[kBatchLdsQueueWord] = 0;
@@ -226,14 +241,15 @@ __global__ __launch_bounds__(kBlock) void BatchBuildKernel(const BatchMesh* __re
             BlockSortPass(even ? keys : ktmp, even ? vals : vtmp, even ? ktmp : keys, even ? vtmp : vals, n,
                           (uint32_t)(p * kSortRadixBits), sh);
         }
-        __syncthreads();  // the hierarchy is emitted by BatchEmitKernel, one thread per node of all meshes
+        ClearTreeCounters(BatchTreeScratch(keys, n), n, tid, kBlock);
+        __syncthreads();  // the tree is built by BatchTreeKernel
     }
 }
 
 // Meshes of at most kBatchLdsMaxTris triangles: one workgroup per mesh
 // computes bounds and Morton codes, runs the four 8-bit passes of the
 // stable sort with keys and values resident in LDS (128 KB for 16,384
-// pairs), and emits the hierarchy from the LDS-resident codes.  Item j of lane l in wave w is position
+// pairs), and writes the sorted pairs out.  Item j of lane l in wave w is position
 // w * (64 * kLdsItems) + 64 j + l, and ranks follow that order (waves, then
 // items, then lanes), so each pass is stable and the result equals the
 // single-mesh sort of the same (code, index) pairs.  kBatchLdsMaxTris is a
@@ -406,36 +422,74 @@ __global__ __launch_bounds__(BLOCK) void BatchBuildLdsKernel(const BatchMesh* __
             }
             __syncthreads();
         }
-        // The hierarchy from the LDS-resident sorted codes (EmitNode, as
-        // EmitHierarchyKernel); BatchRefitKernel refits it.
-        BvhNode* nodes = reinterpret_cast<BvhNode*>(result + sizeof(AccelHeader));
-        for (uint32_t i = tid; i < n; i += kLdsBlock) EmitNode(sh.keys, sh.vals, n, i, nodes);
+        // The sorted codes and primitives, for BatchTreeKernel.
+        uint32_t* keys = RebaseOn<uint32_t>(queue, bm.work);
+        uint32_t* vals = keys + AlignUp(n, 64);
+        for (uint32_t i = tid; i < n; i += kLdsBlock) {
+            keys[i] = sh.keys[i];
+            vals[i] = sh.vals[i];
+        }
+        ClearTreeCounters(BatchTreeScratch(keys, n), n, tid, kLdsBlock);
         // The next mesh's first barrier orders these LDS reads before reuse.
     }
 }
 
-// Karras emission of every mesh, one thread per leaf index (node i and
-// leaf i of its mesh), over the 64-leaf chunks of all meshes: each node's
-// binary searches are a chain of dependent loads, so the whole GPU's
-// threads run them rather than one workgroup per mesh.
-__global__ __launch_bounds__(kBlock) void BatchEmitKernel(const BatchMesh* __restrict__ table, uint32_t meshes,
-                                                          uint32_t total_chunks, uint32_t* scratch) {
-    const uint32_t c = XcdContiguousBlock(blockIdx.x, gridDim.x) * (kBlock / kRefitChunk) + threadIdx.x / kRefitChunk;
-    if (c >= total_chunks) return;
-    uint32_t lo = 0, hi = meshes;  // last mesh with first_chunk <= c (empty meshes own no chunk)
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (table[mid].first_chunk <= c) lo = mid;
-        else hi = mid;
+// The hierarchy and boxes of every mesh (tree_device.h), one thread per leaf
+// over the 64-leaf chunks of all meshes.  The host lays the chunks out so
+// that a mesh of up to kTreeWindow leaves lies in one workgroup and a larger
+// one starts a workgroup of its own: only the mesh at a workgroup's first
+// chunk can have several windows.
+// 2,048 meshes of 64-16,384 triangles (6M in all): 463 us, and 207 us for the
+// two BatchBuildLdsKernels before it; 653 and 515 us when those kernels
+// emitted the hierarchy by binary searches and a refit of all meshes followed.
+__global__ __launch_bounds__(kTreeWindow) void BatchTreeKernel(const BatchMesh* __restrict__ table, uint32_t meshes,
+                                                               uint32_t total_chunks, uint32_t* scratch) {
+    __shared__ TreeLds s;
+    constexpr uint32_t kChunksPerBlock = kTreeWindow / kRefitChunk;
+    static_assert(kChunksPerBlock == kBatchChunksPerWindow, "the host lays chunks out for this kernel");
+    const uint32_t cb = XcdContiguousBlock(blockIdx.x, gridDim.x) * kChunksPerBlock;
+    const uint32_t c = cb + threadIdx.x / kRefitChunk;
+    uint32_t lo_m = 0, hi_m = meshes;  // last mesh with first_chunk <= c (empty meshes own no chunk)
+    while (c < total_chunks && hi_m - lo_m > 1) {
+        const uint32_t mid = (lo_m + hi_m) / 2;
+        if (table[mid].first_chunk <= c) lo_m = mid;
+        else hi_m = mid;
     }
-    const BatchMesh bm = table[lo];
-    const uint32_t i = (c - bm.first_chunk) * kRefitChunk + threadIdx.x % kRefitChunk;
-    if (c < bm.first_chunk || i >= bm.tri_count) return;
+    const BatchMesh bm = table[lo_m];
     const uint32_t n = bm.tri_count;
-    const uint32_t* keys = RebaseOn<const uint32_t>(scratch, bm.work);  // sorted codes after the four passes
-    const uint32_t* vals = keys + AlignUp(n, 64);
+    const uint32_t i = (c - bm.first_chunk) * kRefitChunk + threadIdx.x % kRefitChunk;
+    const bool active = c < total_chunks && c >= bm.first_chunk && i < n;
+    uint32_t* keys = RebaseOn<uint32_t>(scratch, bm.work);
     BvhNode* nodes = reinterpret_cast<BvhNode*>(RebaseOn<uint8_t>(scratch, bm.result) + sizeof(AccelHeader));
-    EmitNode(keys, vals, n, i, nodes);
+    auto code = [keys](int k) { return keys[k]; };
+    float4 q[4];
+    float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {0.0f, 0.0f, 0.0f};
+    uint32_t d = 0, after = 0;
+    if (active) {
+        const uint32_t ci = keys[i];
+        d = (uint32_t)(1 + DeltaOf(code, (int)n, (int)i, ci, (int)i - 1));
+        if (threadIdx.x + 1 == kTreeWindow) after = (uint32_t)(1 + DeltaOf(code, (int)n, (int)i, ci, (int)i + 1));
+        TriangleLeaf(ViewOfBatch(bm, scratch), (keys + AlignUp(n, 64))[i], q, lo, hi);
+    }
+    s.delta_min[0][threadIdx.x] = (uint8_t)d;  // 0 where a mesh starts and where there is none
+    if (threadIdx.x + 1 == kTreeWindow) s.delta_min[0][kTreeWindow] = (uint8_t)after;
+    TreeRun r;
+    const bool waits = BuildWindow(nodes, n, i, active, q, lo, hi, scratch, r, s);
+    // The mesh at the first chunk, if it has more windows than this one.
+    __syncthreads();
+    if (threadIdx.x == 0) s.go = active && TreeWindows(n) > 1 ? lo_m + 1 : 0;
+    __syncthreads();
+    if (s.go == 0) return;
+    const uint32_t m0 = s.go - 1;
+    __syncthreads();
+    const BatchMesh b0 = table[m0];
+    uint32_t* keys0 = RebaseOn<uint32_t>(scratch, b0.work);
+    BvhNode* nodes0 = reinterpret_cast<BvhNode*>(RebaseOn<uint8_t>(scratch, b0.result) + sizeof(AccelHeader));
+    const uint32_t windows = TreeWindows(b0.tri_count);
+    auto code0 = [keys0](int k) { return keys0[k]; };
+    FinishTree(nodes0, b0.tri_count, code0, waits && lo_m == m0, r,
+               CarveTreeScratch(BatchTreeScratch(keys0, b0.tri_count), TreeRuns(windows)),
+               (cb - b0.first_chunk) / kChunksPerBlock, windows, s);
 }
 
 // Refit of every mesh in the table, one thread per leaf: thread t of block b
@@ -498,10 +552,10 @@ uint32_t ResidentBlocks(const void* kernel, int block, int which) {
 }  // namespace
 
 size_t BatchWorkBytes(uint32_t tris) {
-    return std::max(AlignUp(size_t(AlignUp(tris, 64)) * 16, 256), RestructureScratchBytes(tris));
+    return std::max(AlignUp(BatchTreeOffset(tris) + TreeScratchBytes(tris), 256), RestructureScratchBytes(tris));
 }
 
-void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t small, uint32_t big_chunks,
+void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t small,
                 uint32_t total_chunks, void* scratch, hipStream_t s) {
     if (meshes == 0) return;
     big = std::min(big, meshes);
@@ -511,10 +565,6 @@ void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t 
         const uint32_t blocks =
             std::min(big, ResidentBlocks(reinterpret_cast<const void*>(&BatchBuildKernel), kBlock, 0));
         BatchBuildKernel<<<blocks, kBlock, 0, s>>>(table, big, queue);
-        if (big_chunks) {
-            const uint32_t eblocks = (uint32_t)(((uint64_t)big_chunks * kRefitChunk + kBlock - 1) / kBlock);
-            BatchEmitKernel<<<eblocks, kBlock, 0, s>>>(table, big, big_chunks, queue);
-        }
     }
     small = std::min(std::max(small, big), meshes);
     if (small > big) {
@@ -529,7 +579,9 @@ void BatchBuild(const BatchMesh* table, uint32_t meshes, uint32_t big, uint32_t 
             std::min(meshes - small, ResidentBlocks(reinterpret_cast<const void*>(kernel), 256, 2));
         kernel<<<blocks, 256, 0, s>>>(table, small, meshes, queue, kBatchLdsSmallQueueWord);
     }
-    BatchRefit(table, meshes, total_chunks, scratch, s);
+    if (total_chunks)
+        BatchTreeKernel<<<(total_chunks + kBatchChunksPerWindow - 1) / kBatchChunksPerWindow, kTreeWindow, 0, s>>>(
+            table, meshes, total_chunks, queue);
 }
 
 void BatchRefit(const BatchMesh* table, uint32_t meshes, uint32_t total_chunks, void* scratch, hipStream_t s) {

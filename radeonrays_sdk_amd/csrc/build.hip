@@ -7,10 +7,11 @@
 // the TLAS).  The launch structure is this library's own:
 //   init (header, bounds, sort tickets) -> mesh bounds (wave64 reductions,
 //   one set of ordered-uint atomics per block) -> Morton codes fused with the
-//   radix histogram -> onesweep sort -> Karras emission -> refit, where each
-//   finished node writes its box straight into its parent's child slot and
-//   the parity of the parent's `update` counter tells the second arriver to
-//   continue (no reset pass is needed before an update).
+//   radix histogram -> onesweep sort -> the tree with its boxes, in one launch
+//   (tree_device.h).  An update refits: each finished node writes its box
+//   straight into its parent's child slot and the parity of the parent's
+//   `update` counter tells the second arriver to continue (no reset pass is
+//   needed).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,6 +23,7 @@
 #include "build_device.h"
 #include "rr_device.h"
 #include "sort.h"
+#include "tree_device.h"
 
 namespace rr {
 
@@ -47,7 +49,7 @@ struct BuildHead {
 static_assert(sizeof(BuildHead) == 256, "the build head fills its 256-byte scratch slot");
 
 struct BlasScratchLayout {
-    size_t head, keys, vals, keys_tmp, vals_tmp, sort, total;
+    size_t head, keys, vals, keys_tmp, vals_tmp, sort, tree, total;
 };
 
 BlasScratchLayout LayoutBlas(uint32_t n) {
@@ -59,6 +61,7 @@ BlasScratchLayout LayoutBlas(uint32_t n) {
     l.keys_tmp = o; o += AlignUp(size_t(n) * 4, 256);
     l.vals_tmp = o; o += AlignUp(size_t(n) * 4, 256);
     l.sort = o; o += SortScratchBytes(n);
+    l.tree = o; o += AlignUp(TreeScratchBytes(n), 256);
     l.total = o;
     return l;
 }
@@ -180,11 +183,13 @@ __device__ __forceinline__ SceneBounds ReadBounds(const BuildHead* head) {
 }
 
 // Morton code of each primitive's box centroid (lbvh_calc_morton_codes_mesh.comp:78-130),
-// fused with the sort's digit histogram and the clearing of its look-back words.
+// fused with the sort's digit histogram and the clearing of its look-back words
+// and of the tree's arrival counters.
 template <typename CentroidFn>
 __device__ __forceinline__ void MortonAndHistogram(uint32_t n, const BuildHead* head, CentroidFn centroid,
                                                    uint32_t* keys, uint32_t* vals, int passes, uint32_t* sort_hist,
-                                                   uint32_t* sort_status, size_t status_words) {
+                                                   uint32_t* sort_status, size_t status_words, uint32_t* tree_arrived,
+                                                   uint32_t tree_runs) {
     __shared__ uint32_t s_h[kSortMaxPasses][kSortRadix];
     for (uint32_t i = threadIdx.x; i < kSortMaxPasses * kSortRadix; i += kBlock) (&s_h[0][0])[i] = 0;
     const SceneBounds b = ReadBounds(head);
@@ -209,44 +214,57 @@ __device__ __forceinline__ void MortonAndHistogram(uint32_t n, const BuildHead* 
     }
     for (size_t w = (size_t)blockIdx.x * kBlock + threadIdx.x; w < status_words; w += (size_t)gridDim.x * kBlock)
         sort_status[w] = 0;
+    for (uint32_t w = blockIdx.x * kBlock + threadIdx.x; w < tree_runs; w += gridDim.x * kBlock) tree_arrived[w] = 0;
 }
 
 __global__ __launch_bounds__(kBlock) void MeshMortonKernel(MeshView m, const BuildHead* head, uint32_t* keys,
                                                            uint32_t* vals, int passes, uint32_t* sort_hist,
-                                                           uint32_t* sort_status, size_t status_words) {
+                                                           uint32_t* sort_status, size_t status_words,
+                                                           uint32_t* tree_arrived, uint32_t tree_runs) {
     auto centroid = [&](uint32_t t, float c[3]) { TriangleCentroid(m, t, c); };
-    MortonAndHistogram(m.tri_count, head, centroid, keys, vals, passes, sort_hist, sort_status, status_words);
+    MortonAndHistogram(m.tri_count, head, centroid, keys, vals, passes, sort_hist, sort_status, status_words, tree_arrived,
+                       tree_runs);
 }
 
-// Block b emits nodes [256 b, 256 b + 256).  Its codes and kEmitMargin
-// codes on either side are staged in LDS: most nodes have short key
-// ranges, so most probes of their searches read LDS; the others read
-// memory.  Same codes either way, so the same tree.
-constexpr int kEmitMargin = 256;
-constexpr int kEmitWindow = kBlock + 2 * kEmitMargin;
-__global__ __launch_bounds__(kBlock) void EmitHierarchyKernel(const uint32_t* __restrict__ codes,
-                                                              const uint32_t* __restrict__ prims, uint32_t n,
-                                                              BvhNode* __restrict__ nodes) {
-    __shared__ uint32_t s_codes[kEmitWindow];
-    const int lo = (int)(blockIdx.x * kBlock) - kEmitMargin;
-    for (int k = threadIdx.x; k < kEmitWindow; k += kBlock) {
-        const int g = lo + k;
-        s_codes[k] = (g >= 0 && g < (int)n) ? codes[g] : 0u;
+// The hierarchy over the sorted codes with its boxes (tree_device.h), one
+// leaf per thread.  `leaf` gives leaf i's quads, all but the parent link, and
+// its box.  1,045,458 triangles: 100 us, 1.9 TB/s of vertices, codes and nodes
+// (52 us for the top-down emission and 97 us for the refit that it replaces);
+// 333,333: 53 us (27 + 57).  What is left are the windows' steps through LDS
+// (three workgroups per CU) and two hand-offs of about 12 us.
+template <typename Leaf>
+__device__ __forceinline__ void BuildTree(BvhNode* __restrict__ nodes, uint32_t n, const uint32_t* __restrict__ codes,
+                                          void* tree, const Leaf& leaf) {
+    __shared__ TreeLds s;
+    const uint32_t windows = gridDim.x;
+    // Neighbouring windows share an XCD's L2 for the triangles they read.
+    const uint32_t window = XcdContiguousBlock(blockIdx.x, windows);
+    const uint32_t i = window * kTreeWindow + threadIdx.x;
+    auto code = [codes](int k) { return codes[k]; };
+    const bool active = i < n;
+    float4 q[4];
+    float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {0.0f, 0.0f, 0.0f};
+    uint32_t d = 0;
+    if (active) {
+        const uint32_t c = codes[i];
+        d = (uint32_t)(1 + DeltaOf(code, (int)n, (int)i, c, (int)i - 1));
+        if (threadIdx.x + 1 == kTreeWindow)
+            s.delta_min[0][kTreeWindow] = (uint8_t)(1 + DeltaOf(code, (int)n, (int)i, c, (int)i + 1));
+        leaf(i, q, lo, hi);
+    } else if (threadIdx.x + 1 == kTreeWindow) {
+        s.delta_min[0][kTreeWindow] = 0;
     }
-    __syncthreads();
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    // An LDS read always (clamped index) and a memory read only outside the
-    // window, kept as two loads: one select between the two addresses would
-    // become a flat load.
-    auto code = [&](int k) -> uint32_t {
-        const uint32_t o = (uint32_t)(k - lo);
-        const bool in = o < (uint32_t)kEmitWindow;
-        uint32_t v = s_codes[in ? o : 0u];
-        if (!in) v = LdG(codes + k);
-        return v;
-    };
-    EmitNodeWith(code, prims, n, i, nodes);
+    s.delta_min[0][threadIdx.x] = (uint8_t)d;
+    TreeRun r;
+    const bool waits = BuildWindow(nodes, n, i, active, q, lo, hi, nodes, r, s);
+    if (windows > 1) FinishTree(nodes, n, code, waits, r, CarveTreeScratch(tree, TreeRuns(windows)), window, windows, s);
+}
+
+__global__ __launch_bounds__(kTreeWindow) void BuildTreeKernel(MeshView m, const uint32_t* __restrict__ codes,
+                                                               const uint32_t* __restrict__ prims, void* tree,
+                                                               BvhNode* __restrict__ nodes) {
+    BuildTree(nodes, m.tri_count, codes, tree,
+              [&](uint32_t i, float4 q[4], float lo[3], float hi[3]) { TriangleLeaf(m, prims[i], q, lo, hi); });
 }
 
 // One thread per leaf; block b's leaves (key positions [256 b, 256 b + 256))
@@ -985,7 +1003,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void Ba
 constexpr float kInstanceBoxWiden = 1.52587890625e-05f;  // 2^-16
 
 struct TlasScratchLayout {
-    size_t upload, head, boxes, keys, vals, keys_tmp, vals_tmp, sort, total;
+    size_t upload, head, boxes, keys, vals, keys_tmp, vals_tmp, sort, tree, total;
 };
 TlasScratchLayout LayoutTlas(uint32_t n) {
     TlasScratchLayout l;
@@ -998,6 +1016,7 @@ TlasScratchLayout LayoutTlas(uint32_t n) {
     l.keys_tmp = o; o += AlignUp(size_t(n) * 4, 256);
     l.vals_tmp = o; o += AlignUp(size_t(n) * 4, 256);
     l.sort = o; o += SortScratchBytes(n);
+    l.tree = o; o += AlignUp(TreeScratchBytes(n), 256);
     l.total = o;
     return l;
 }
@@ -1088,7 +1107,7 @@ __global__ __launch_bounds__(kBlock) void TlasInstanceKernel(const InstanceUploa
 __global__ __launch_bounds__(kBlock) void TlasMortonKernel(const float* __restrict__ boxes, uint32_t n,
                                                            const BuildHead* head, uint32_t* keys, uint32_t* vals,
                                                            int passes, uint32_t* sort_hist, uint32_t* sort_status,
-                                                           size_t status_words) {
+                                                           size_t status_words, uint32_t* tree_arrived, uint32_t tree_runs) {
     auto centroid = [&](uint32_t t, float c[3]) {
         const float4 lo = reinterpret_cast<const float4*>(boxes)[2 * (size_t)t];
         const float4 hi = reinterpret_cast<const float4*>(boxes)[2 * (size_t)t + 1];
@@ -1096,7 +1115,26 @@ __global__ __launch_bounds__(kBlock) void TlasMortonKernel(const float* __restri
         c[1] = (lo.y + hi.y) * 0.5f;
         c[2] = (lo.z + hi.z) * 0.5f;
     };
-    MortonAndHistogram(n, head, centroid, keys, vals, passes, sort_hist, sort_status, status_words);
+    MortonAndHistogram(n, head, centroid, keys, vals, passes, sort_hist, sort_status, status_words, tree_arrived, tree_runs);
+}
+
+// As BuildTreeKernel over instances; a leaf stores its instance's world box
+// twice (lbvh_fit_aabb_scene.comp:125-128).
+__global__ __launch_bounds__(kTreeWindow) void BuildSceneTreeKernel(const float* __restrict__ boxes, uint32_t n,
+                                                                    const uint32_t* __restrict__ codes,
+                                                                    const uint32_t* __restrict__ ids, void* tree,
+                                                                    BvhNode* __restrict__ nodes) {
+    BuildTree(nodes, n, codes, tree, [&](uint32_t i, float4 q[4], float lo[3], float hi[3]) {
+        const uint32_t id = ids[i];
+        const float4 blo = reinterpret_cast<const float4*>(boxes)[2 * (size_t)id];
+        const float4 bhi = reinterpret_cast<const float4*>(boxes)[2 * (size_t)id + 1];
+        q[0] = make_float4(blo.x, blo.y, blo.z, __uint_as_float(kInvalid));
+        q[1] = make_float4(bhi.x, bhi.y, bhi.z, __uint_as_float(id));
+        q[2] = make_float4(blo.x, blo.y, blo.z, 0.0f);
+        q[3] = make_float4(bhi.x, bhi.y, bhi.z, __uint_as_float(0u));
+        lo[0] = blo.x; lo[1] = blo.y; lo[2] = blo.z;
+        hi[0] = bhi.x; hi[1] = bhi.y; hi[2] = bhi.z;
+    });
 }
 
 // One thread per instance leaf; block b's leaves form one refit window.
@@ -1190,13 +1228,15 @@ void BuildBlas(const MeshDesc& mesh, bool restructure, void* scratch, void* resu
     uint32_t* keys = At<uint32_t>(scratch, L.keys);
     uint32_t* vals = At<uint32_t>(scratch, L.vals);
     const int passes = SortPasses(30);
-    MeshMortonKernel<<<Blocks(n), kBlock, 0, s>>>(m, head, keys, vals, passes, sc.hist, sc.status, sc.status_words);
+    const uint32_t windows = TreeWindows(n);
+    void* tree = At<void>(scratch, L.tree);
+    MeshMortonKernel<<<Blocks(n), kBlock, 0, s>>>(m, head, keys, vals, passes, sc.hist, sc.status, sc.status_words,
+                                                  static_cast<uint32_t*>(tree), windows > 1 ? TreeRuns(windows) : 0);
     const bool in_place = RadixSortPairs(keys, vals, At<uint32_t>(scratch, L.keys_tmp), At<uint32_t>(scratch, L.vals_tmp),
                                          n, 30, sc, true, s);
     const uint32_t* sk = in_place ? keys : At<uint32_t>(scratch, L.keys_tmp);
     const uint32_t* sv = in_place ? vals : At<uint32_t>(scratch, L.vals_tmp);
-    EmitHierarchyKernel<<<Blocks(n), kBlock, 0, s>>>(sk, sv, n, nodes);
-    LaunchMeshRefit(m, result, s);
+    BuildTreeKernel<<<windows, kTreeWindow, 0, s>>>(m, sk, sv, tree, nodes);
     if (do_restructure) RestructureBlas(n, scratch, result, s);
 }
 
@@ -1339,14 +1379,16 @@ void BuildTlas(const InstanceUpload* instances, uint32_t n, void* scratch, void*
                                                     At<uint64_t>(result, table_off), boxes, head);
     uint32_t* keys = At<uint32_t>(scratch, L.keys);
     uint32_t* vals = At<uint32_t>(scratch, L.vals);
+    const uint32_t windows = TreeWindows(n);
+    void* tree = At<void>(scratch, L.tree);
     TlasMortonKernel<<<Blocks(n), kBlock, 0, s>>>(boxes, n, head, keys, vals, SortPasses(30), sc.hist, sc.status,
-                                                  sc.status_words);
+                                                  sc.status_words, static_cast<uint32_t*>(tree),
+                                                  windows > 1 ? TreeRuns(windows) : 0);
     const bool in_place = RadixSortPairs(keys, vals, At<uint32_t>(scratch, L.keys_tmp), At<uint32_t>(scratch, L.vals_tmp),
                                          n, 30, sc, true, s);
     const uint32_t* sk = in_place ? keys : At<uint32_t>(scratch, L.keys_tmp);
     const uint32_t* sv = in_place ? vals : At<uint32_t>(scratch, L.vals_tmp);
-    EmitHierarchyKernel<<<Blocks(n), kBlock, 0, s>>>(sk, sv, n, nodes);
-    RefitSceneKernel<<<Blocks(n), kBlock, 0, s>>>(boxes, n, nodes);
+    BuildSceneTreeKernel<<<windows, kTreeWindow, 0, s>>>(boxes, n, sk, sv, tree, nodes);
 }
 
 }  // namespace rr

@@ -56,8 +56,8 @@ __device__ __forceinline__ void TriangleCentroid(const MeshView& m, uint32_t t, 
     }
 }
 
-// Karras 2012 binary radix tree over sorted codes
-// (lbvh_emit_hierarchy_mesh.comp:85-217).  delta(i, j) is the common prefix
+// Prefix lengths of the binary radix tree over sorted codes (Karras 2012,
+// lbvh_emit_hierarchy_mesh.comp:85-217).  delta(i, j) is the common prefix
 // length of codes i and j, with 32 + clz(i ^ j) for equal codes and -1 for
 // j outside [0, n).  `code(k)` returns sorted code k (from memory, or from a
 // copy in LDS); ci = code(i).
@@ -68,58 +68,7 @@ __device__ __forceinline__ int DeltaOf(const Code& code, int n, int i, uint32_t 
     return ci != b ? __clz(ci ^ b) : 32 + __clz((uint32_t)(i ^ j));
 }
 
-// Node i's topology (and leaf i's primitive) from the sorted codes: Karras
-// 2012.  A leaf's other words (its vertices or box, child0 = kInvalid,
-// update = 0) are written by the refit that follows every emission
-// (WriteLeaf, RefitSceneKernel), which reads child1 and parent from here.
-template <typename Code>
-__device__ __forceinline__ void EmitNodeWith(const Code& code, const uint32_t* __restrict__ prims, uint32_t n,
-                                             uint32_t i, BvhNode* __restrict__ nodes) {
-    const uint32_t leaf = n - 1 + i;
-    nodes[leaf].child1 = prims[i];
-    if (n == 1) {
-        nodes[0].parent = kInvalid;
-        return;
-    }
-    if (i >= n - 1) return;
-    const int N = (int)n, I = (int)i;
-    const uint32_t ci = code(I);
-    // Direction and far end of node i's key range.
-    const int d = (DeltaOf(code, N, I, ci, I + 1) - DeltaOf(code, N, I, ci, I - 1)) > 0 ? 1 : -1;
-    const int dmin = DeltaOf(code, N, I, ci, I - d);
-    int lmax = 2;
-    while (DeltaOf(code, N, I, ci, I + lmax * d) > dmin) lmax *= 2;
-    int l = 0;
-    for (int t = lmax / 2; t >= 1; t /= 2)
-        if (DeltaOf(code, N, I, ci, I + (l + t) * d) > dmin) l += t;
-    const int j = I + l * d;
-    const int first = min(I, j), last = max(I, j);
-    // Split: last position that shares more than the range's common prefix with `first`.
-    const uint32_t cf = code(first);
-    const int common = DeltaOf(code, N, first, cf, last);
-    int lo = first, hi = last;
-    while (hi > lo + 1) {
-        const int mid = (lo + hi) / 2;
-        if (DeltaOf(code, N, first, cf, mid) > common) lo = mid;
-        else hi = mid;
-    }
-    const int split = lo;
-    const uint32_t left = (split == first) ? (n - 1 + (uint32_t)split) : (uint32_t)split;
-    const uint32_t right = (split + 1 == last) ? (n - 1 + (uint32_t)split + 1) : (uint32_t)split + 1;
-    nodes[i].child0 = left;
-    nodes[i].child1 = right;
-    nodes[i].update = 0;
-    nodes[left].parent = i;
-    nodes[right].parent = i;
-    if (i == 0) nodes[0].parent = kInvalid;
-}
-
-__device__ __forceinline__ void EmitNode(const uint32_t* __restrict__ codes, const uint32_t* __restrict__ prims,
-                                         uint32_t n, uint32_t i, BvhNode* __restrict__ nodes) {
-    EmitNodeWith([codes](int k) { return codes[k]; }, prims, n, i, nodes);
-}
-
-// Bottom-up refit shared by BLAS build/update and TLAS build
+// Bottom-up refit of the updates of BLASes and scenes
 // (lbvh_fit_aabb_mesh.comp:122-205, lbvh_fit_aabb_scene.comp:98-167).  Each
 // finished node stores its box into its parent's child slot, then bumps the
 // parent's arrival counter (wrapping from 1 back to 0); a previous value of
@@ -138,11 +87,16 @@ __device__ __forceinline__ void WaitStores() { asm volatile("s_waitcnt vmcnt(0)"
 // store or load with the cache policy of agent-scope relaxed atomic accesses
 // (sc1: written through, read past stale lines), one memory transaction per
 // side instead of three.  The loads wait for their data before returning.
+// A store of more than 64 bits reads its data registers up to two wait states
+// after it issues.  The compiler keeps that distance for its own stores, but
+// knows nothing of one in inline asm and may overwrite the registers at once,
+// so each such store brings its wait states along.
+#define RR_STORE_WAIT_STATES "\n\ts_nop 2"
 typedef float RrBox3 __attribute__((ext_vector_type(3)));
 __device__ __forceinline__ void StoreBoxAgent(float* p, float x, float y, float z) {
     RrBox3 v;
     v.x = x; v.y = y; v.z = z;
-    asm volatile("global_store_dwordx3 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx3 %0, %1, off sc1" RR_STORE_WAIT_STATES : : "v"(p), "v"(v) : "memory");
 }
 // A whole node (four 16-byte quads), agent-scope, waited for.
 __device__ __forceinline__ void LoadNodeAgent(const BvhNode* nd, float4& q0, float4& q1, float4& q2, float4& q3) {
@@ -214,6 +168,20 @@ __device__ __forceinline__ void ClimbRefit(BvhNode* __restrict__ nodes, uint32_t
         p = up;
         c0 = nc0;
         up = nup;
+    }
+}
+
+// The quads of a new leaf, all but its parent link: triangle prim; gives its box.
+__device__ __forceinline__ void TriangleLeaf(const MeshView& m, uint32_t prim, float4 q[4], float lo[3], float hi[3]) {
+    float v[9];
+    LoadTriangle(m, prim, v);
+    q[0] = make_float4(v[0], v[1], v[2], __uint_as_float(kInvalid));
+    q[1] = make_float4(v[3], v[4], v[5], __uint_as_float(prim));
+    q[2] = make_float4(v[6], v[7], v[8], 0.0f);
+    q[3] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(0u));
+    for (int a = 0; a < 3; ++a) {
+        lo[a] = fminf(fminf(v[a], v[3 + a]), v[6 + a]);
+        hi[a] = fmaxf(fmaxf(v[a], v[3 + a]), v[6 + a]);
     }
 }
 
