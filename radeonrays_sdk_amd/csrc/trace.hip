@@ -270,9 +270,9 @@ __device__ __forceinline__ void WriteHit(void* __restrict__ hits, uint32_t i, bo
 // The grid holds only as many waves as the GPU keeps resident.  Rays are split
 // into kQueues contiguous ranges, one per XCD (workgroups are dispatched to
 // the XCDs round-robin), so that neighbouring rays share an L2; each wave
-// takes 64 ray indices at a time from its range with one atomic and hands
-// them to lanes as their rays finish, moving on to the other ranges once its
-// own is empty.  Each lane runs a while-while loop (Aila & Laine, "Understanding
+// starts with a piece of its range, takes further pieces with one atomic each
+// and hands the rays to lanes as theirs finish, moving on to the other ranges
+// once its own is empty.  Each lane runs a while-while loop (Aila & Laine, "Understanding
 // the Efficiency of Ray Traversal on GPUs", HPG 2009): inner nodes until every
 // busy lane holds a postponed leaf, then the leaves.  Leaves are still tested
 // in depth-first order, so closest and any hits are those of the plain
@@ -296,19 +296,57 @@ __device__ __forceinline__ void InitQueues(uint32_t* counters, uint32_t n) {
     __syncthreads();
 }
 
+// A wave's view of the ray queues (wave-uniform): rays [next, end) are its
+// own, and it takes `piece` more at a time from queue q.
+struct RayQueue {
+    uint32_t next, end, q, piece;
+    uint32_t tries;  // queues found empty
+    bool drained;    // no more rays to take
+};
+
+// The rays at the head of queue q that the waves starting on it have from
+// the beginning, a piece each: its counter counts those behind them.
+__device__ __forceinline__ uint32_t QueueFirst(uint32_t q, uint32_t piece) {
+    return (gridDim.x + kQueues - 1 - q) / kQueues * (kBlock / 64) * piece;
+}
+
 // A wave's first rays.  When the grid's lanes hold every ray, each wave has
-// an equal share of them from the start and takes none from the queues
-// (true; its rays are [q_next, q_end), at most one per lane).
-__device__ __forceinline__ bool StartQueue(uint32_t n, uint32_t& q, uint32_t& q_next, uint32_t& q_end) {
-    q = blockIdx.x % kQueues;
-    q_next = q_end = 0;
+// an equal share of them, at most one per lane, and takes none from the
+// queues (true); else its piece at the head of its queue, without an atomic
+// (all waves at once would wait for each other's: 4M rays of a camera above
+// the 1M-triangle terrain 506 -> 491 us, 4M rays towards a 3,000-triangle
+// soup 337 -> 330).
+__device__ __forceinline__ bool StartQueue(RayQueue& s, uint32_t n, uint32_t part, uint32_t fetch) {
     const uint32_t waves = gridDim.x * (kBlock / 64);
     const uint32_t share = n / waves + (n % waves != 0);
-    if (share > 64) return false;
-    const uint32_t w = XcdContiguousBlock(blockIdx.x, gridDim.x) * (kBlock / 64) + threadIdx.x / 64;
-    q_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)min((uint64_t)w * share, (uint64_t)n));
-    q_end = q_next + min(share, n - q_next);
-    return true;
+    const bool fixed = share <= 64;
+    s.q = blockIdx.x % kQueues;
+    s.piece = fixed ? share : fetch;
+    s.tries = 0;
+    const uint32_t block = fixed ? XcdContiguousBlock(blockIdx.x, gridDim.x) : blockIdx.x / kQueues;
+    const uint32_t first = fixed ? 0 : s.q * part, end = fixed ? n : min((s.q + 1) * part, n);
+    const uint32_t w = block * (kBlock / 64) + threadIdx.x / 64;
+    s.next = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)min(first + (uint64_t)w * s.piece, (uint64_t)end));
+    s.end = s.next + min(s.piece, end - s.next);
+    s.drained = fixed && s.next == s.end;
+    return fixed;
+}
+
+// Takes the next piece, from the next queue that has any once its own is empty.
+__device__ __forceinline__ void TakeRays(RayQueue& s, uint32_t* counters, uint32_t n, uint32_t part) {
+    while (!s.drained) {
+        uint32_t b = 0;
+        if (__lane_id() == 0) b = atomicAdd(&counters[s.q * kQueueStride], s.piece);
+        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + QueueFirst(s.q, s.piece);
+        const uint32_t end = min((s.q + 1) * part, n);
+        if (b < end) {
+            s.next = b;
+            s.end = min(b + s.piece, end);
+            return;
+        }
+        s.drained = ++s.tries == kQueues;
+        s.q = s.q + 1 == kQueues ? 0 : s.q + 1;
+    }
 }
 
 // First spill word of a wave: its lanes' slots, or with equal shares, where
@@ -329,23 +367,29 @@ __device__ __forceinline__ size_t SpillStart(bool fixed, uint32_t first_ray) {
 // node in each step while 64 are left.  A ray's state stays in its lane's
 // registers and is shuffled to the lanes that work for it.
 //
-// The list is in depth-first order from the top: lanes take entries in that
-// order and their children replace them in that order (near child first).
-// Any hit needs it: the first hit in depth-first order wins, so a hit
-// cancels what its ray has below it (later in that order), and a hit found
-// above it afterwards replaces it.  Closest hits do not depend on the order.
+// A ray's entries are in depth-first order from the top: lanes take entries in
+// that order and their children replace them in that order (near child
+// first).  Any hit needs it: the first hit in depth-first order wins, so a
+// hit cancels what its ray has below it (later in that order), and a hit
+// found above it afterwards replaces it.  Closest hits do not depend on the
+// order.  Entries of different rays mix freely, and PoolPush puts each ray's
+// next one above everyone's far children: in one depth-first list the top
+// 64 entries were a few rays' far subtrees, visited before the near ones
+// could cull them (32 camera rays in a 65,536-triangle soup: 98 nodes a ray
+// and 54 steps, now 49 and 29; 131,072 such rays 186 -> 118 us, 1M-triangle
+// terrain 190 -> 121, scene of 1,000 instances 1265 -> 1084).
 //
 // What bounds it: the chain of node fetches, a tree's depth of steps of one
 // memory round trip each; with many rays left also VALU issue (a step is
 // about 130 instructions, 64 entries at once, where the lanes' own loop
 // spends a node's on a quarter of its lanes).  4M incoherent rays over the
-// 1M-triangle terrain: closest 574 -> 462 us, any 532 -> 407 us, against
+// 1M-triangle terrain: closest 574 -> 451 us, any 532 -> 399 us, against
 // lanes that traverse (closest hit: and split) their rays alone to the end;
-// 1,000 rays 111 -> 32 us.  The list takes the stacks' LDS; 72 VGPRs leave
+// 1,000 rays 111 -> 33 us.  The list takes the stacks' LDS; 72 VGPRs leave
 // seven waves per SIMD instead of eight (held to 64 it spills, and was
 // slower: 529 us), which costs long rays less than the end of the launch
-// gains (65,536-triangle soup, 4M rays from inside: 2524 -> 2430, any
-// 1889 -> 1747 us).
+// gains (65,536-triangle soup, 4M rays from inside: 2524 -> 2401, any
+// 1889 -> 1740 us).
 //
 // An entry is (node, slot | depth << 6): the lane that holds the ray, and
 // how many entries the ray's own stack would hold when the node is popped
@@ -391,30 +435,80 @@ __device__ __forceinline__ bool PoolFits(const LaneStack<DEPTH>& st, uint32_t no
     return (uint32_t)__builtin_amdgcn_readlane((int)sum, 63) + kPoolReserve <= (uint32_t)kPoolCapacity<DEPTH>;
 }
 
+// A pool shorter than this goes on with as many rays as it has (PoolPush); a
+// longer one finishes some first, or it would outgrow its room and shrink to
+// few entries a step (64 long rays a wave: a batch of 32 requests 1240 us,
+// without this limit 1300; a quarter or three quarters of the room instead
+// of half: 262,144 camera rays over the terrain 215 and 143 against 154 us,
+// the 1,000-instance scene 1073 and 1408 against 1084).
+template <int DEPTH>
+constexpr uint32_t kPoolWide = (kPoolCapacity<DEPTH> - kPoolReserve) / 2;
+
 // Turns the wave's stacks into the pool, in place: lane 0's entries on top,
-// each lane's in the order of its stack.  Returns the number of entries.
+// each lane's in the order of its stack (a short pool: every ray's first
+// entry above everyone's others).  Returns the number of entries.
 template <int DEPTH>
 __device__ __forceinline__ uint32_t PoolFromStacks(uint32_t (*lds)[64], uint32_t sp, uint32_t node, uint32_t leaf,
                                                    uint32_t rid) {
     const uint32_t lane = __lane_id();
     const uint32_t entries = rid != kInvalid ? sp : 0u;
-    const uint32_t sum = WavePrefixSum(PoolOwn(sp, node, leaf, rid));
+    uint32_t sum = WavePrefixSum(PoolOwn(sp, node, leaf, rid));
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+    const bool lead = total < kPoolWide<DEPTH> && rid != kInvalid && (node != kInvalid || leaf != kInvalid);
+    const uint64_t leads = __ballot(lead);
+    sum -= RankIn(leads) + (lead ? 1u : 0u);
+    const uint32_t rest = total - (uint32_t)__popcll(leads);
     uint32_t row[DEPTH];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) row[i] = lds[i][lane];
     WaveLdsFence();
-    uint2* at = reinterpret_cast<uint2*>(lds) + (total - sum);
+    uint2* at = reinterpret_cast<uint2*>(lds) + (rest - sum);
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) {
         __builtin_amdgcn_sched_barrier(0);  // one entry's second word at a time in registers
         if ((uint32_t)i < entries) at[i] = make_uint2(row[i], lane | (uint32_t)i << kPoolSlotBits);
     }
     at += entries;
-    if (rid != kInvalid && node != kInvalid) *at++ = make_uint2(node, lane | entries << kPoolSlotBits);
-    if (rid != kInvalid && leaf != kInvalid) *at = make_uint2(leaf, lane | entries << kPoolSlotBits);
+    const uint32_t word = lane | entries << kPoolSlotBits;
+    if (rid != kInvalid && node != kInvalid && (leaf != kInvalid || !lead)) *at++ = make_uint2(node, word);
+    if (rid != kInvalid && leaf != kInvalid && !lead) *at = make_uint2(leaf, word);
+    if (lead) reinterpret_cast<uint2*>(lds)[total - 1 - RankIn(leads)] = make_uint2(leaf != kInvalid ? leaf : node, word);
     WaveLdsFence();
     return total;
+}
+
+// Pushes a step's children: on top the first one of each ray (closest hit:
+// every near child), so that the next step goes on with as many rays as
+// there are, and their far children are left until the near ones are done
+// and may have made them needless; below them the rest, in the order of the
+// entries they came from.  A ray's own entries stay in depth-first order
+// (closest hit does not need it).  With the list half full, all in order:
+// that keeps it short.
+template <bool CLOSEST>
+__device__ __forceinline__ void PoolPush(uint2* pool, uint32_t& count, uint32_t wide, uint32_t* first, uint32_t step, int slot,
+                                         uint32_t near, uint32_t near_word, uint32_t far, uint32_t far_word) {
+    const uint32_t lane = __lane_id();
+    bool lead = false;
+    if (count < wide) {
+        lead = near != kInvalid;
+        if (!CLOSEST) {
+            // The lowest lane with a child of this ray.
+            const uint32_t key = step << 6 | (63u - lane);
+            if (lead) atomicMax(&first[slot], key);
+            WaveLdsFence();
+            lead = lead && first[slot] == key;
+        }
+    }
+    const uint64_t m0 = __ballot(lead), m1 = __ballot(near != kInvalid && !lead), m2 = __ballot(far != kInvalid);
+    const uint32_t rest = count + (uint32_t)(__popcll(m1) + __popcll(m2));
+    const uint32_t below = RankIn(m1) + RankIn(m2);
+    if (near != kInvalid) {
+        const uint32_t at = lead ? rest + (uint32_t)__popcll(m0) - 1 - RankIn(m0) : rest - 1 - below;
+        pool[at] = make_uint2(near, near_word);
+    }
+    if (far != kInvalid) pool[rest - 1 - below - (near != kInvalid && !lead ? 1u : 0u)] = make_uint2(far, far_word);
+    WaveLdsFence();
+    count = rest + (uint32_t)__popcll(m0);
 }
 
 // A lane's best hit while the pool is worked on (in LDS: read and written
@@ -423,6 +517,7 @@ struct PoolHits {
     float t[64];  // any hit: the hit's distance (the ray's best_t stays its t_max)
     float u[64], v[64];
     uint32_t prim[64];
+    uint32_t first[64];  // PoolPush
 };
 
 // The geometry a pool's entries belong to: one for the launch, or (batched
@@ -439,8 +534,13 @@ enum PoolKind : int { kPoolClosest = 0, kPoolAny = 1, kPoolPerLane = 2 };
 // for any hit); best.prim starts as the best hit so far.
 template <int KIND, int DEPTH>
 __device__ __forceinline__ void PoolTraverse(uint2* pool, uint32_t count, const PoolBvh& bvh, const RayState& own,
-                                             float& best_t, PoolHits& best, uint32_t* err) {
+                                             float& best_t, PoolHits& best, uint32_t* first, uint32_t* err) {
     const uint32_t lane = __lane_id();
+    uint32_t step = 0;
+    if (KIND != kPoolClosest) {
+        first[lane] = 0;
+        WaveLdsFence();
+    }
     constexpr uint32_t kRoom = kPoolCapacity<DEPTH> - kPoolReserve;
     constexpr uint32_t kSlotMask = (1u << kPoolSlotBits) - 1;
     while (count) {
@@ -530,13 +630,8 @@ __device__ __forceinline__ void PoolTraverse(uint2* pool, uint32_t count, const 
                 WaveLdsFence();
             }
         }
-        const uint64_t m0 = __ballot(near != kInvalid), m1 = __ballot(far != kInvalid);
-        const uint32_t pushed = (uint32_t)(__popcll(m0) + __popcll(m1));
-        const uint32_t top = count + pushed - 1 - RankIn(m0) - RankIn(m1);
-        if (near != kInvalid) pool[top] = make_uint2(near, e.y + (far != kInvalid ? 1u << kPoolSlotBits : 0u));
-        if (far != kInvalid) pool[top - 1] = make_uint2(far, e.y);
-        WaveLdsFence();
-        count += pushed;
+        PoolPush<KIND == kPoolClosest>(pool, count, kPoolWide<DEPTH>, first, ++step, slot, near,
+                                       e.y + (far != kInvalid ? 1u << kPoolSlotBits : 0u), far, e.y);
     }
 }
 
@@ -563,9 +658,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     const uint32_t part = (n + kQueues - 1) / kQueues;
 
     // Wave-uniform queue state.
-    uint32_t q, tries = 0, q_next, q_end;
-    const bool fixed = StartQueue(n, q, q_next, q_end);
-    bool drained = fixed && q_next == q_end;
+    RayQueue rq;
+    const bool fixed = StartQueue(rq, n, part, fetch);
     bool pooled = false;  // the wave's last rays go on in a pool
 
     // Lane state.
@@ -578,33 +672,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     float any_limit = 0.0f;  // any hit: the culling limit, fixed per ray (the first hit ends the ray)
     uint32_t best_prim = kInvalid;
     uint32_t node = kInvalid, leaf = kInvalid;
-    LaneStack<DEPTH> st{s_stack[threadIdx.x / 64], scratch + kQueueHeadWords + SpillStart(fixed, q_next), err, 0, 0};
+    LaneStack<DEPTH> st{s_stack[threadIdx.x / 64], scratch + kQueueHeadWords + SpillStart(fixed, rq.next), err, 0, 0};
     for (;;) {
         // Refill idle lanes.
         const uint64_t idle = __ballot(rid == kInvalid);
-        if (idle && !drained) {
-            if (q_next == q_end) {
-                for (;;) {
-                    uint32_t b = 0;
-                    if (lane == 0) b = atomicAdd(&counters[q * kQueueStride], fetch);
-                    b = __shfl(b, 0, 64);
-                    const uint32_t end = min((q + 1) * part, n);
-                    if (b < end) {
-                        q_next = b;
-                        q_end = min(b + fetch, end);
-                        break;
-                    }
-                    if (++tries == kQueues) {
-                        drained = true;
-                        break;
-                    }
-                    q = q + 1 == kQueues ? 0 : q + 1;
-                }
-            }
-            const uint32_t take = min((uint32_t)__popcll(idle), q_end - q_next);
+        if (idle && !rq.drained) {
+            if (rq.next == rq.end) TakeRays(rq, counters, n, part);
+            const uint32_t take = min((uint32_t)__popcll(idle), rq.end - rq.next);
             const uint32_t rank = RankIn(idle);
             if (rid == kInvalid && rank < take) {
-                rid = q_next + rank;
+                rid = rq.next + rank;
                 const RayIn ray = LoadRay(rays, rid);
                 SetupRay(r, ray.a.x, ray.a.y, ray.a.z, ray.a.w, ray.b.x, ray.b.y, ray.b.z);
                 best_t = ray.b.w;
@@ -615,14 +692,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 node = total ? 0u : kInvalid;
                 leaf = kInvalid;
             }
-            q_next += take;
-            if (fixed) drained = true;  // a share is at most one ray per lane
+            rq.next += take;
+            if (fixed) rq.drained = true;  // a share is at most one ray per lane
         }
         if (__ballot(rid != kInvalid) == 0) {
-            if (drained) break;
+            if (rq.drained) break;
             continue;
         }
-        if (drained && PoolFits(st, node, leaf, rid)) {
+        if (rq.drained && PoolFits(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -657,7 +734,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 }
                 // Leave for the leaf phase once every descending lane holds a
                 // leaf, or once too few lanes are still descending.
-                if (!__any(leaf == kInvalid) || (!drained && (uint32_t)__popcll(__ballot(1)) < min_busy)) break;
+                if (!__any(leaf == kInvalid) || (!rq.drained && (uint32_t)__popcll(__ballot(1)) < min_busy)) break;
             }
             // Phase B: the postponed leaf, then any leaves that come next in order.
             if (leaf == kInvalid && node != kInvalid && node >= n_int) {
@@ -698,9 +775,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 rid = kInvalid;
                 break;
             }
-            if (!drained && (uint32_t)__popcll(__ballot(1)) < min_busy) break;  // refill (nothing left once drained)
+            if (!rq.drained && (uint32_t)__popcll(__ballot(1)) < min_busy) break;  // refill (nothing left once rq.drained)
             // Drained, but the pool had no room: try again once a lane is done.
-            if (drained && __ballot(1) != entered) break;
+            if (rq.drained && __ballot(1) != entered) break;
         }
     }
     // The wave's last rays.
@@ -712,7 +789,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
         best.prim[lane] = best_prim;
         WaveLdsFence();
         PoolTraverse<ANY ? kPoolAny : kPoolClosest, DEPTH>(reinterpret_cast<uint2*>(st.lds), count,
-                                                           PoolBvh{nodes, n_int, total, boxes, ANY}, r, best_t, best, err);
+                                                           PoolBvh{nodes, n_int, total, boxes, ANY}, r, best_t, best, best.first, err);
         if (rid != kInvalid) {
             best_prim = best.prim[lane];
             const bool hit = best_prim != kInvalid;
@@ -740,8 +817,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
 // transforms it again, as entering the instance does, so each step costs
 // that and one more dependent load (the instance's BLAS address), against
 // one step per node of a ray's whole chain.  Every BLAS's nodes follow its
-// header.  1,000 instances of 2,000-triangle soups, 262,144 any-hit rays:
-// 1258 -> 906 us; 40,000 closest-hit rays 1.43 -> 0.49 ms.
+// header.  A scene of 1,000 instances of 2,000-triangle soups built and
+// traced: 262,144 any-hit rays 1.70 -> 1.08 ms, 40,000 closest-hit rays
+// 1.44 -> 0.46 ms.
 constexpr uint32_t kPoolDepthBits = 7;
 constexpr uint32_t kPoolInstShift = kPoolSlotBits + kPoolDepthBits;
 constexpr uint32_t kPoolWorld = (1u << (32 - kPoolInstShift)) - 1;  // and the number of instances a pool can name
@@ -756,13 +834,17 @@ __device__ __forceinline__ uint32_t PoolFromStacks2L(uint32_t (*lds)[64], uint32
                                                      uint32_t cur_total) {
     const uint32_t lane = __lane_id();
     const uint32_t entries = rid != kInvalid ? sp : 0u;
-    const uint32_t sum = WavePrefixSum(PoolOwn(sp, node, leaf, rid));
+    uint32_t sum = WavePrefixSum(PoolOwn(sp, node, leaf, rid));
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+    const bool lead = total < kPoolWide<DEPTH> && rid != kInvalid && (node != kInvalid || leaf != kInvalid);
+    const uint64_t leads = __ballot(lead);
+    sum -= RankIn(leads) + (lead ? 1u : 0u);
+    const uint32_t rest = total - (uint32_t)__popcll(leads);
     uint32_t row[DEPTH];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) row[i] = lds[i][lane];
     WaveLdsFence();
-    uint2* at = reinterpret_cast<uint2*>(lds) + (total - sum);
+    uint2* at = reinterpret_cast<uint2*>(lds) + (rest - sum);
     uint32_t level = lane | kPoolWorld << kPoolInstShift, limit = top_total;
     const uint32_t in = lane | (inst == kInvalid ? kPoolWorld : inst) << kPoolInstShift;
 #pragma unroll
@@ -778,9 +860,11 @@ __device__ __forceinline__ uint32_t PoolFromStacks2L(uint32_t (*lds)[64], uint32
         }
     }
     at += entries;
-    if (rid != kInvalid && node != kInvalid)
-        *at++ = make_uint2(node == kTopLevelSentinel ? kInvalid : node, in | entries << kPoolSlotBits);
-    if (rid != kInvalid && leaf != kInvalid) *at = make_uint2(leaf, in | entries << kPoolSlotBits);
+    const uint32_t word = in | entries << kPoolSlotBits;
+    const uint32_t top = node == kTopLevelSentinel ? kInvalid : node;
+    if (rid != kInvalid && node != kInvalid && (leaf != kInvalid || !lead)) *at++ = make_uint2(top, word);
+    if (rid != kInvalid && leaf != kInvalid && !lead) *at = make_uint2(leaf, word);
+    if (lead) reinterpret_cast<uint2*>(lds)[total - 1 - RankIn(leads)] = make_uint2(leaf != kInvalid ? leaf : top, word);
     WaveLdsFence();
     return total;
 }
@@ -795,8 +879,13 @@ struct PoolScene {
 template <bool ANY, int DEPTH>
 __device__ __forceinline__ void PoolTraverse2L(uint2* pool, uint32_t count, const PoolScene& top, const float (*world)[kBlock],
                                                float tmin, float& best_t, float& hit_t, float& bu, float& bv,
-                                               uint32_t& best_prim, uint32_t& best_inst, uint32_t* err) {
+                                               uint32_t& best_prim, uint32_t& best_inst, uint32_t* first, uint32_t* err) {
     const uint32_t lane = __lane_id();
+    uint32_t step = 0;
+    if (ANY) {
+        first[lane] = 0;
+        WaveLdsFence();
+    }
     const uint32_t wave0 = threadIdx.x & ~63u;
     constexpr uint32_t kRoom = kPoolCapacity<DEPTH> - kPoolReserve;
     constexpr uint32_t kSlotMask = (1u << kPoolSlotBits) - 1, kDepthMask = (1u << kPoolDepthBits) - 1;
@@ -904,13 +993,7 @@ __device__ __forceinline__ void PoolTraverse2L(uint2* pool, uint32_t count, cons
                 if ((cancelled >> (pool[i].y & kSlotMask)) & 1ull) pool[i].x = kInvalid;
             WaveLdsFence();
         }
-        const uint64_t m0 = __ballot(near != kInvalid), m1 = __ballot(far != kInvalid);
-        const uint32_t pushed = (uint32_t)(__popcll(m0) + __popcll(m1));
-        const uint32_t at = count + pushed - 1 - RankIn(m0) - RankIn(m1);
-        if (near != kInvalid) pool[at] = make_uint2(near, next);
-        if (far != kInvalid) pool[at - 1] = make_uint2(far, e.y);
-        WaveLdsFence();
-        count += pushed;
+        PoolPush<!ANY>(pool, count, kPoolWide<DEPTH>, first, ++step, slot, near, next, far, e.y);
     }
 }
 
@@ -928,6 +1011,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     // with a fresh set-up), so the watertight shear and axis permutation of
     // the world ray are not kept.
     __shared__ float s_world[9][kBlock];
+    __shared__ uint32_t s_first[kBlock / 64][64];  // PoolPush
     uint32_t n = ray_count;
     if (indirect) n = min(n, *indirect);
     if (init_queues) InitQueues(scratch, n);
@@ -944,9 +1028,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     const uint32_t part = (n + kQueues - 1) / kQueues;
 
     // Wave-uniform queue state.
-    uint32_t q, tries = 0, q_next, q_end;
-    const bool fixed = StartQueue(n, q, q_next, q_end);
-    bool drained = fixed && q_next == q_end;
+    RayQueue rq;
+    const bool fixed = StartQueue(rq, n, part, fetch);
     bool pooled = false;  // the wave's last rays go on in a pool
 
     // Lane state: the ray of the level being traversed (the world ray waits
@@ -961,34 +1044,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     const BvhNode* cur = top_nodes;
     uint32_t cur_int = top_int, cur_total = top_total;
     bool boxes = false;
-    LaneStack<DEPTH> st{s_stack[threadIdx.x / 64], scratch + kQueueHeadWords + SpillStart(fixed, q_next), err, 0, 0};
+    LaneStack<DEPTH> st{s_stack[threadIdx.x / 64], scratch + kQueueHeadWords + SpillStart(fixed, rq.next), err, 0, 0};
 
     for (;;) {
         // Refill idle lanes.
         const uint64_t idle = __ballot(rid == kInvalid);
-        if (idle && !drained) {
-            if (q_next == q_end) {
-                for (;;) {
-                    uint32_t b = 0;
-                    if (lane == 0) b = atomicAdd(&counters[q * kQueueStride], fetch);
-                    b = __shfl(b, 0, 64);
-                    const uint32_t end = min((q + 1) * part, n);
-                    if (b < end) {
-                        q_next = b;
-                        q_end = min(b + fetch, end);
-                        break;
-                    }
-                    if (++tries == kQueues) {
-                        drained = true;
-                        break;
-                    }
-                    q = q + 1 == kQueues ? 0 : q + 1;
-                }
-            }
-            const uint32_t take = min((uint32_t)__popcll(idle), q_end - q_next);
+        if (idle && !rq.drained) {
+            if (rq.next == rq.end) TakeRays(rq, counters, n, part);
+            const uint32_t take = min((uint32_t)__popcll(idle), rq.end - rq.next);
             const uint32_t rank = RankIn(idle);
             if (rid == kInvalid && rank < take) {
-                rid = q_next + rank;
+                rid = rq.next + rank;
                 const RayIn ray = LoadRay(rays, rid);
                 s_world[0][threadIdx.x] = ray.a.x; s_world[1][threadIdx.x] = ray.a.y; s_world[2][threadIdx.x] = ray.a.z;
                 s_world[3][threadIdx.x] = ray.b.x; s_world[4][threadIdx.x] = ray.b.y; s_world[5][threadIdx.x] = ray.b.z;
@@ -1007,14 +1073,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 node = top_total ? 0u : kInvalid;
                 leaf = kInvalid;
             }
-            q_next += take;
-            if (fixed) drained = true;  // a share is at most one ray per lane
+            rq.next += take;
+            if (fixed) rq.drained = true;  // a share is at most one ray per lane
         }
         if (__ballot(rid != kInvalid) == 0) {
-            if (drained) break;
+            if (rq.drained) break;
             continue;
         }
-        if (drained && top_prims < kPoolWorld && PoolFits(st, node, leaf, rid)) {
+        if (rq.drained && top_prims < kPoolWorld && PoolFits(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -1099,7 +1165,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 }
                 // An index past the level's nodes (corrupt buffer) ends the ray.
                 if (node != kInvalid && node != kTopLevelSentinel && node >= cur_total) node = kInvalid;
-                if (!__any(leaf == kInvalid) || (!drained && (uint32_t)__popcll(__ballot(1)) < min_busy)) break;
+                if (!__any(leaf == kInvalid) || (!rq.drained && (uint32_t)__popcll(__ballot(1)) < min_busy)) break;
             }
             // Phase B: the postponed leaf, then the leaves that follow it in order.
             if (leaf == kInvalid && inst != kInvalid && node >= cur_int && node < cur_total) {
@@ -1142,9 +1208,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                 leaf = kInvalid;
                 break;
             }
-            if (!drained && (uint32_t)__popcll(__ballot(1)) < min_busy) break;  // refill (nothing left once drained)
+            if (!rq.drained && (uint32_t)__popcll(__ballot(1)) < min_busy) break;  // refill (nothing left once rq.drained)
             // Drained, but the pool had no room: try again once a lane is done.
-            if (drained && __ballot(1) != entered) break;
+            if (rq.drained && __ballot(1) != entered) break;
         }
     }
     // The wave's last rays.
@@ -1154,7 +1220,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
         float hit_t = best_t;
         PoolTraverse2L<ANY, DEPTH>(reinterpret_cast<uint2*>(st.lds), count,
                                    PoolScene{top_nodes, xforms, blas_table, top_total, top_prims}, s_world, r.tmin, best_t,
-                                   hit_t, bu, bv, best_prim, best_inst, err);
+                                   hit_t, bu, bv, best_prim, best_inst, s_first[threadIdx.x / 64], err);
         if (rid != kInvalid)
             WriteHit<OUT, true>(hits, rid, best_prim != kInvalid, bu, bv, best_inst, best_prim, ANY ? hit_t : best_t, best_t);
     }
@@ -1416,7 +1482,7 @@ __global__ __launch_bounds__(kBlock) void TraceBatchKernel(const BatchRequest* _
         WaveLdsFence();
         PoolTraverse<kPoolPerLane, kLdsStackEntries>(reinterpret_cast<uint2*>(st.lds), count,
                                                      PoolBvh{nodes, n_int, total, boxes, (lflags & 1u) != 0}, r, best_t,
-                                                     best, err);
+                                                     best, best.first, err);
         if (rid != kInvalid) {
             best_prim = best.prim[lane];
             const bool hit = best_prim != kInvalid;
@@ -1811,12 +1877,16 @@ uint32_t QueryBlocks(uint64_t n, bool two, bool shares = false) {
 uint32_t BatchBlocks() { return ResidentBlocks(reinterpret_cast<const void*>(&TraceBatchKernel), 1); }
 uint32_t Batch2LBlocks() { return ResidentBlocks(reinterpret_cast<const void*>(&TraceBatch2LKernel), 7); }
 
-// Rays per queue atomic for n rays over `blocks` blocks: the level's tuned
-// value, cut (to a multiple of 32, at least 32) when fewer rays than waves x
-// fetch would leave waves without any.
+// Rays per piece for n rays over `blocks` blocks: the level's tuned value, at
+// most half an even share (as a multiple of 32, at least 32), so that waves
+// whose rays end early find more to take (524,288 rays of a camera, closest
+// hit: 65,536-triangle soup 331 -> 235 us, 1M-triangle terrain 253 -> 211).
+// Smaller ones still cost more in atomics than they balance (1M rays in
+// pieces of 64: terrain 292 -> 227 us, but 3,000-triangle soup 158 -> 172,
+// and 4M rays 330 -> 374).
 uint32_t FetchFor(uint32_t n, uint32_t blocks, bool two) {
     const uint64_t waves = (uint64_t)blocks * (kBlock / 64);
-    const uint64_t per = (n + waves - 1) / waves;
+    const uint64_t per = (n + 2 * waves - 1) / (2 * waves);
     const uint32_t f = (uint32_t)std::max<uint64_t>(32, (per + 31) / 32 * 32);
     return std::min(two ? RaysPerFetch2L() : RaysPerFetch(), f);
 }

@@ -113,3 +113,27 @@ def test_pooled_shares_follow_the_device_count(ctx, dev, world, limit):
     if live:
         assert torch.equal(hits[:live * 16], _plain(ctx, world["soup"], rays[:live], "closest", "full"))
     assert bool((hits[live * 16:] == 0xAB).all())
+
+
+@pytest.mark.parametrize("fetch", [32, 64, 128])
+@pytest.mark.parametrize("which,extra", [("soup", 1), ("soup", 8 * 64 * 128 + 5), ("scene", 37)])
+def test_pieces_hand_out_every_ray_once(ctx, dev, world, which, extra, fetch):
+    """More rays than equal shares hold: a first piece per wave, the rest from the queues; an indirect count cuts the
+    queues shorter than the pieces were sized for."""
+    n = SHARED + extra
+    say(f"queue pieces, {which}, {n} rays, {fetch} a piece")
+    key = rr.RRX_TUNING_TRACE_2L_RAYS_PER_FETCH if which == "scene" else rr.RRX_TUNING_TRACE_RAYS_PER_FETCH
+    saved = autotune.get(ctx.lib, key)
+    rays = to_dev(_soup_rays(n, 15), dev)
+    want = _plain(ctx, world[which], rays, "closest", "full")
+    for live in (n, SHARED + 1):
+        count = torch.tensor([live], dtype=torch.int32, device=dev)
+        hits = torch.full((n * 16,), 0xAB, dtype=torch.uint8, device=dev)
+        try:
+            autotune.set_(ctx.lib, key, fetch)
+            ctx.intersect(world[which], rays, "closest", "full", indirect=count, hits=hits)
+            torch.cuda.synchronize()
+        finally:
+            autotune.set_(ctx.lib, key, saved)
+        assert torch.equal(hits[:live * 16], want[:live * 16]), live
+        assert bool((hits[live * 16:] == 0xAB).all()), live
