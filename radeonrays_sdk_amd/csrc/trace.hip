@@ -1838,11 +1838,15 @@ uint32_t PersistentBlocks(bool two) {
 // tree is deep, so more waves with fewer rays each are faster until the
 // SIMDs are full.  Closest / any in microseconds, 65,536-triangle soup,
 // rays from inside, one ray per lane before -> equal shares: 1,000 rays
-// 202/228 -> 33/32, 16,000 222/287 -> 54/53, 131,072 349/416 -> 186/168;
-// 1M-triangle terrain, 131,072 rays 190/206 -> 52/50.  16 waves per CU
-// against 4, 8 and 32: 131,072 rays 186 us against 265, 233 and 211 (soup),
-// 52 against 95, 55 and 53 (terrain).  The grid may have more lanes than
-// rays (SpillStart).
+// 202/228 -> 30/31, 16,000 222/287 -> 53/49, 131,072 349/416 -> 129/122;
+// 1M-triangle terrain, 131,072 rays 190/206 -> 46/47.  16 waves per CU
+// against 24: 262,144 rays from inside the soup 198 against 246, camera rays
+// 183 against 150 (terrain: 60 against 63, 145 against 144); 64 rays each
+// for up to 28 waves gains as much on some queries (393,216 rays, terrain:
+// from inside 112 -> 83) as it loses on others (camera 168 -> 188).  A
+// scene's rays are longer: 24 waves per CU (1,000 instances built and
+// 262,144 rays traced: 1074 -> 945 us; 300 instances, 180,000 rays: 148 ->
+// 118).  The grid may have more lanes than rays (SpillStart).
 //
 // Otherwise never more than one ray per lane and never more
 // than four workgroups per CU (four waves per SIMD) unless 512 x k rays per
@@ -1850,7 +1854,7 @@ uint32_t PersistentBlocks(bool two) {
 // the single-level kernel takes a workgroup per 256 x k rays, at least one
 // per CU; the two-level kernel, whose rays are four times longer, keeps one
 // ray per lane.  k = 0: the full grid whenever the rays fill it.
-constexpr uint32_t kSharedWaves = 16;
+constexpr uint32_t kSharedWaves = 16, kSharedWaves2L = 24;
 uint32_t QueryBlocks(uint64_t n, bool two, bool shares = false) {
     const uint64_t one_per_lane = std::max<uint64_t>(1, (n + kBlock - 1) / kBlock);
     const uint32_t k = RaysPerLane();
@@ -1866,7 +1870,7 @@ uint32_t QueryBlocks(uint64_t n, bool two, bool shares = false) {
         cus = (uint32_t)std::max(1, c);
         cus_of[dev].store(cus, std::memory_order_relaxed);
     }
-    const uint64_t shared_waves = (uint64_t)cus * kSharedWaves;
+    const uint64_t shared_waves = (uint64_t)cus * (two ? kSharedWaves2L : kSharedWaves);
     if (shares && n <= shared_waves * 64) return (uint32_t)std::min<uint64_t>((n + 3) / 4, shared_waves / 4);
     const uint64_t lo = two ? one_per_lane : (n + (uint64_t)kBlock * k - 1) / ((uint64_t)kBlock * k);
     const uint64_t hi = (n + (uint64_t)kBlock * 2 * k - 1) / ((uint64_t)kBlock * 2 * k);
