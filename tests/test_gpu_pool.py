@@ -137,3 +137,16 @@ def test_pieces_hand_out_every_ray_once(ctx, dev, world, which, extra, fetch):
             autotune.set_(ctx.lib, key, saved)
         assert torch.equal(hits[:live * 16], want[:live * 16]), live
         assert bool((hits[live * 16:] == 0xAB).all()), live
+
+
+@pytest.mark.parametrize("sizes", [(1,), (64, 65, 1), (0, 3, 0, 130) * 30, (97,) * 700, (256,) * 1700])
+def test_batch_chunks_are_found_among_any_number_of_requests(ctx, dev, world, sizes):
+    """One chunk to more chunks than the grid has waves; the request of a chunk is searched 64 at a time."""
+    say(f"batched requests, {len(sizes)} of {max(sizes)} rays")
+    rays = to_dev(_soup_rays(max(sizes), 16), dev)
+    want = {(w, q): _plain(ctx, world[w], rays, q, "full") for w in ("soup", "dup") for q in ("closest", "any")}
+    picks = [(("soup", "dup")[k % 2], ("closest", "any")[k // 2 % 2]) for k in range(len(sizes))]
+    got = ctx.intersect_batch([(world[w], rays[:n], q, "full") for n, (w, q) in zip(sizes, picks)])
+    torch.cuda.synchronize()
+    for k, (hits, n, pick) in enumerate(zip(got, sizes, picks)):
+        assert n == 0 or torch.equal(hits[:16 * n], want[pick][:16 * n]), (k, pick)
