@@ -69,14 +69,15 @@ BlasScratchLayout LayoutBlas(uint32_t n) {
 // Treelet restructuring scratch (reuses the key/value region of the LBVH
 // scratch, which is dead once the hierarchy is emitted).
 struct RestructureLayout {
-    size_t counter, roots, counts, total;
+    size_t counter, roots, counts, total;  // a counter and counts of n nodes per round
 };
+constexpr int kRestructureRounds = 3;
 __host__ __device__ RestructureLayout LayoutRestructure(uint32_t n) {
     RestructureLayout l;
     size_t o = 0;
     l.counter = o; o += 256;
     l.roots = o; o += AlignUp(size_t(n) * 4, 256);
-    l.counts = o; o += AlignUp(size_t(NodeCount(n)) * 4, 256);
+    l.counts = o; o += AlignUp(size_t(n) * kRestructureRounds * 4, 256);
     l.total = o;
     return l;
 }
@@ -356,10 +357,13 @@ __device__ __forceinline__ void StU(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(kBlock) void InitTreeletCountsKernel(uint32_t n, uint32_t* counts, uint32_t* counter) {
+// Every round's counts and counter in one launch (three cost 4.6 us each for a
+// small mesh).
+__global__ __launch_bounds__(kBlock) void InitTreeletCountsKernel(uint32_t n, uint32_t* counts, uint32_t* counters) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n - 1) counts[i] = 0;
-    if (i == 0) *counter = 0;
+    if (i < n)
+        for (int r = 0; r < kRestructureRounds; ++r) counts[(size_t)r * n + i] = 0;
+    if (i < kRestructureRounds) counters[i] = 0;
 }
 
 // Climb from each leaf, accumulating primitive counts; the first node whose
@@ -526,9 +530,15 @@ __global__ __launch_bounds__(kBlock) void FindTreeletRootsKernel(const BvhNode* 
     for (uint32_t k = threadIdx.x; k < cnt; k += kBlock) roots[s_base + k] = s_roots[k];
 }
 
-// One wave per treelet root.  Lane 0 does the pointer-chasing parts (forming
-// the treelet, rewiring it, climbing); the 128 subset areas and the dynamic
-// programme over subsets run across the wave.
+// One wave per treelet root.  The wave fetches the nodes around the root and
+// forms the treelet from wave-uniform values, the 128 subset areas and the
+// dynamic programme over subsets run across it, lane 0 rewires and climbs.
+// What bounds it: the chain of passes up the tree, each a chain itself (three
+// levels of fetches, six steps of the programme, the rewiring, the hand-off).
+// With lane 0 opening one node after another, five dependent loads and their
+// choices through LDS, and a launch per round to clear the counts: 997
+// triangles 266 -> 237 us for the whole build, 65,536 697 -> 619, 1,045,458
+// 1262 -> 1156; a batch of 300 meshes restructured 3.36 -> 3.29 ms.
 // The body runs for one root of one BVH (nodes, n leaves, arrival counts
 // of its internal nodes); the single-mesh and batched kernels call it.
 template <int LEAVES, bool kFiveLeafGroups>
@@ -538,7 +548,6 @@ __device__ __forceinline__ void RestructureFromRoot(BvhNode* nodes, uint32_t n, 
     __shared__ uint32_t s_leaf[kTreeletLeaves];
     __shared__ uint32_t s_inner[kTreeletLeaves - 1];
     __shared__ float s_box[kTreeletLeaves][6];
-    __shared__ float s_leaf_area[kTreeletLeaves];
     __shared__ float s_area[kTreeletMasks];
     // Box of each leaf subset (lo xyz, hi xyz), kept from step 2 for the
     // rewiring; not for 9-leaf treelets, whose 512 boxes would take 12 KB
@@ -547,62 +556,119 @@ __device__ __forceinline__ void RestructureFromRoot(BvhNode* nodes, uint32_t n, 
     __shared__ float s_sbox[kSubsetBoxes ? kTreeletMasks : 1][6];
     __shared__ float s_cost[kTreeletMasks];
     __shared__ uint32_t s_part[kTreeletMasks];
-    __shared__ uint32_t s_root;
-    __shared__ uint32_t s_parent;
-    __shared__ uint32_t s_go;
-    const uint32_t lane = threadIdx.x;
+    uint32_t lane = threadIdx.x;
     const uint32_t n_int = n - 1;
-    if (lane == 0) s_root = root;
-    __syncthreads();
+    // Fetched nodes, one per lane: lanes 0-13 the three levels below the root
+    // (level l in lanes 2^l - 2 and up), the root and its parent in lanes 14
+    // and 15 or 15 and 14, from 16 on nodes opened deeper than that.
+    float4 q0, q1, q2, q3;
+    float area0 = 0.0f, area1 = 0.0f;  // of the two child boxes
+    constexpr uint32_t kFetched = 14;
+    uint32_t root_lane = kFetched;
+    const auto fetch = [&](uint32_t at) {
+        LoadNodeAgent(nodes + at, q0, q1, q2, q3);
+        float b0[6], b1[6];
+        SlotBoxes(q0, q1, q2, q3, b0, b1);
+        area0 = SurfaceArea(b0, b0 + 3);
+        area1 = SurfaceArea(b1, b1 + 3);
+    };
+    if (lane == root_lane) fetch(root);
     // Each pass moves one level up, so a tree of n leaves needs fewer than n passes.
     for (uint32_t pass = 0; pass < n; ++pass) {
+        // Held to 64 VGPRs (the batched kernel): what depends on the lane alone
+        // is not kept in registers over a pass.
+        if (!kFiveLeafGroups) asm volatile("" : "+v"(lane));
         // 1. Form a treelet: repeatedly open the treelet leaf with the largest
         //    surface area (restructure_bvh.comp:170-218).
         //    A node's two child boxes are in its own slots (exact unions,
         //    kept current by refit and by every finished treelet), so opening
-        //    a node is one load of that node: its child links and both boxes.
-        if (lane == 0) {
-            const uint32_t root = s_root;
-            float* area = s_leaf_area;  // LDS: indexed at run time (registers would spill)
-            float (*box)[6] = s_box;
-            s_inner[0] = root;
-            float4 q0, q1, q2, q3;
-            LoadNodeAgent(nodes + root, q0, q1, q2, q3);
-            s_parent = __float_as_uint(q2.w);
-            s_leaf[0] = __float_as_uint(q0.w);
-            s_leaf[1] = __float_as_uint(q1.w);
-            SlotBoxes(q0, q1, q2, q3, box[0], box[1]);
-            area[0] = SurfaceArea(box[0], box[0] + 3);
-            area[1] = SurfaceArea(box[1], box[1] + 3);
-            bool ok = s_leaf[0] < 2 * n - 1 && s_leaf[1] < 2 * n - 1;
-            for (int size = 2; ok && size < kTreeletLeaves; ++size) {
-                float largest = 0.0f;
-                int sel = -1;
-                for (int k = 0; k < size; ++k) {
-                    if (s_leaf[k] < n_int && (largest == 0.0f || area[k] > largest)) {
-                        largest = area[k];
-                        sel = k;
-                    }
-                }
-                if (sel < 0) { ok = false; break; }
-                const uint32_t opened = s_leaf[sel];
-                s_inner[size - 1] = opened;
-                LoadNodeAgent(nodes + opened, q0, q1, q2, q3);
-                const uint32_t c0 = __float_as_uint(q0.w), c1 = __float_as_uint(q1.w);
-                if (c0 >= 2 * n - 1 || c1 >= 2 * n - 1) { ok = false; break; }
-                s_leaf[sel] = c0;
-                s_leaf[size] = c1;
-                SlotBoxes(q0, q1, q2, q3, box[sel], box[size]);
-                area[sel] = SurfaceArea(box[sel], box[sel] + 3);
-                area[size] = SurfaceArea(box[size], box[size] + 3);
+        //    a node takes that node alone: its child links and both boxes.
+        //    The three levels below the root are fetched first, a level at a
+        //    time, and the choice is made on wave-uniform values; the root
+        //    itself was fetched in the pass below it, with its children (its
+        //    links and boxes do not change before the hand-off).
+        const auto lane_u = [](float v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (int)l); };
+        const uint32_t parent = lane_u(q2.w, root_lane);
+        for (uint32_t level = 1; level <= 3; ++level) {
+            const uint32_t first = (1u << level) - 2, k = lane - first;
+            const uint32_t up = level == 1 ? root_lane : (first >> 1) - 1 + ((k >> 1) & 7u);
+            const uint32_t c0 = (uint32_t)__shfl((int)__float_as_uint(q0.w), (int)up, 64);
+            const uint32_t c1 = (uint32_t)__shfl((int)__float_as_uint(q1.w), (int)up, 64);
+            if (k < 1u << level) {
+                const uint32_t at = k & 1u ? c1 : c0;
+                if (at < n_int) fetch(at);
+                else q0.w = q1.w = __uint_as_float(kInvalid);
+            } else if (level == 1 && lane == (root_lane ^ 1u) && parent < n_int) {
+                fetch(parent);
             }
-            s_go = ok ? 1u : 0u;
+        }
+        uint32_t leaf[kTreeletLeaves], from[kTreeletLeaves], own[kTreeletLeaves];  // index, 2 x lane of its parent + which, its lane
+        float area[kTreeletLeaves];
+        uint32_t inner[kTreeletLeaves - 1];
+        leaf[0] = lane_u(q0.w, root_lane);
+        leaf[1] = lane_u(q1.w, root_lane);
+        area[0] = __uint_as_float(lane_u(area0, root_lane));
+        area[1] = __uint_as_float(lane_u(area1, root_lane));
+        from[0] = 2 * root_lane;
+        from[1] = 2 * root_lane + 1;
+        own[0] = 0;
+        own[1] = 1;
+        uint32_t deeper = kFetched + 2;
+        bool ok = leaf[0] < 2 * n - 1 && leaf[1] < 2 * n - 1;
+#pragma unroll
+        for (int size = 2; size < kTreeletLeaves; ++size) {
+            float largest = 0.0f;
+            int sel = -1;
+            uint32_t opened = kInvalid, at = kFetched;
+#pragma unroll
+            for (int k = 0; k < size; ++k) {
+                if (leaf[k] < n_int && (largest == 0.0f || area[k] > largest)) {
+                    largest = area[k];
+                    sel = k;
+                    opened = leaf[k];
+                    at = own[k];
+                }
+            }
+            ok = ok && sel >= 0;
+            if (ok && at >= kFetched) {
+                at = deeper++;
+                if (lane == at) fetch(opened);
+            }
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ok ? at : root_lane));
+            const uint32_t c0 = lane_u(q0.w, at), c1 = lane_u(q1.w, at);
+            ok = ok && c0 < 2 * n - 1 && c1 < 2 * n - 1;
+            const float a0 = __uint_as_float(lane_u(area0, at)), a1 = __uint_as_float(lane_u(area1, at));
+            const uint32_t below = at < kFetched / 2 - 1 ? 2 * at + 2 : kFetched;  // the two children's lanes
+#pragma unroll
+            for (int k = 0; k < size; ++k) {
+                const bool here = k == sel;
+                leaf[k] = here ? c0 : leaf[k];
+                area[k] = here ? a0 : area[k];
+                from[k] = here ? 2 * at : from[k];
+                own[k] = here ? below : own[k];
+            }
+            leaf[size] = c1;
+            area[size] = a1;
+            from[size] = 2 * at + 1;
+            own[size] = below < kFetched ? below + 1 : kFetched;
+            inner[size - 1] = opened;
+        }
+        inner[0] = root;
+#pragma unroll
+        for (int k = 0; k < kTreeletLeaves; ++k) {
+            if (lane == 0) s_leaf[k] = leaf[k];
+            if (lane == 0 && k < kTreeletLeaves - 1) s_inner[k] = inner[k];
+            if (lane == from[k] >> 1) {
+                const float b[2][6] = {{q0.x, q0.y, q0.z, q1.x, q1.y, q1.z}, {q2.x, q2.y, q2.z, q3.x, q3.y, q3.z}};
+                for (int a = 0; a < 6; ++a) s_box[k][a] = from[k] & 1u ? b[1][a] : b[0][a];
+            }
         }
         __syncthreads();
-        if (s_go) {
+        if (ok) {
             // 2. Surface area of every subset of the 7 treelet leaves.
             for (uint32_t m = lane; m < kTreeletMasks; m += 64) {
                 float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+#pragma unroll(kFiveLeafGroups ? kTreeletLeaves : 1)
                 for (int k = 0; k < kTreeletLeaves; ++k)
                     if (m & (1u << k))
                         for (int a = 0; a < 3; ++a) {
@@ -866,23 +932,16 @@ __device__ __forceinline__ void RestructureFromRoot(BvhNode* nodes, uint32_t n, 
         //    atomic, and the second arriver then reads what the first wrote.
         //    The root's parent link was read with the root in step 1 (no
         //    other wave writes it before this hand-off).
-        if (lane == 0) {
-            const uint32_t parent = s_parent;
-            uint32_t go = 0;
-            if (parent < n_int) {
-                WaitStores();
-                const uint32_t old =
-                    __hip_atomic_fetch_add(&counts[parent], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (old != 0) {
-                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                    s_root = parent;
-                    go = 1;
-                }
-            }
-            s_go = go;
+        uint32_t old = 0;
+        if (lane == 0 && parent < n_int) {
+            WaitStores();
+            old = __hip_atomic_fetch_add(&counts[parent], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
         }
         __syncthreads();
-        if (!s_go) return;
+        if (__builtin_amdgcn_readfirstlane((int)old) == 0) return;
+        root = parent;
+        root_lane ^= 1u;
     }
 }
 
@@ -1314,8 +1373,8 @@ void RestructureBlas(uint32_t n, void* scratch, void* result, hipStream_t s) {
     uint32_t* roots = At<uint32_t>(scratch, L.roots);
     uint32_t* counts = At<uint32_t>(scratch, L.counts);
     uint32_t min_prims = 64;  // restructure_hlbvh.cpp:34-35,151,276: 64, 128, 256
-    for (int round = 0; round < 3; ++round, min_prims *= 2) {
-        InitTreeletCountsKernel<<<Blocks(n), kBlock, 0, s>>>(n, counts, counter);
+    InitTreeletCountsKernel<<<Blocks(n), kBlock, 0, s>>>(n, counts, counter);
+    for (int round = 0; round < kRestructureRounds; ++round, min_prims *= 2, ++counter, counts += n) {
         FindTreeletRootsKernel<<<Blocks(n), kBlock, 0, s>>>(nodes, n, min_prims, counts, counter, roots);
         const dim3 grid(Blocks(n, (int)min_prims));
         switch (TreeletLeaves()) {
