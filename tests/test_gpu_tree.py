@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import oracle
-from radeonrays_sdk_amd import scenes
+from radeonrays_sdk_amd import autotune, rr, scenes
 from tests.gpu_util import nodes_equal, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +66,28 @@ def test_batched_trees_share_windows(ctx, dev):
     for k, ((v, i), a) in enumerate(zip(meshes, accels)):
         ok, msg = nodes_equal(a.buffer.cpu().numpy(), oracle.build_blas(v, i, False))
         assert ok, f"mesh {k} (n={sizes[k]}): {msg}"
+
+
+@pytest.mark.parametrize("leaves", [5, 7, 9])
+@pytest.mark.parametrize("kind", ["soup", "growing"])
+def test_treelets_opened_deeper_than_the_fetched_levels(ctx, dev, kind, leaves):
+    """Restructured nodes equal the oracle's; triangles whose sizes grow along their order make treelets that open
+    one side again and again, below the three levels fetched with a treelet's root."""
+    n = 3000
+    say(f"treelets of {leaves} leaves, {kind}")
+    v, i = scenes.triangle_soup(n, scenes.rng_for(71, leaves))
+    if kind == "growing":
+        c = np.stack([np.arange(n) / n] * 3, axis=1)
+        size = 1e-5 * 1.5 ** (np.arange(n) % 29)
+        tri = np.array([[-1, 0, 0.3], [1, 0.2, 0], [0, 1, -0.3]])
+        v = (c[:, None, :] + size[:, None, None] * tri).astype(np.float32).reshape(-1, 3)
+        i = np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+    saved = autotune.get(ctx.lib, rr.RRX_TUNING_TREELET_LEAVES)
+    try:
+        autotune.set_(ctx.lib, rr.RRX_TUNING_TREELET_LEAVES, leaves)
+        accel = ctx.build_geometry(to_dev(v, dev), to_dev(i, dev), restructure=True)
+        torch.cuda.synchronize()
+    finally:
+        autotune.set_(ctx.lib, rr.RRX_TUNING_TREELET_LEAVES, saved)
+    ok, msg = nodes_equal(accel.buffer.cpu().numpy(), oracle.build_blas(v, i, True, leaves))
+    assert ok, msg
