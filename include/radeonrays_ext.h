@@ -74,7 +74,8 @@ RR_API RRError rrxCmdIntersectWithStats(RRContext        context,
 typedef enum RRxTuning
 {
     RRX_TUNING_TRACE_MIN_BUSY = 0,        /* refill a wave once fewer lanes traverse (1..64; default 24) */
-    RRX_TUNING_TRACE_RAYS_PER_FETCH = 1,  /* ray indices per queue atomic (32, 64, 128; default 128) */
+    RRX_TUNING_TRACE_RAYS_PER_FETCH = 1,  /* rays a wave takes at a time (32, 64, 128; default 128; at
+                                             most half an even share, at least 32) */
     RRX_TUNING_TRACE_LDS_STACK = 2,       /* LDS stack entries per lane (8, 16, 32; default 16) */
     RRX_TUNING_TRACE_PLAIN = 3,           /* 1: one lane per ray for its whole traversal, no
                                              persistent kernels (default 0, or 1 when the
@@ -100,14 +101,14 @@ typedef enum RRxTuning
                                              concentrated in a few buckets sort slower.  0 (default):
                                              the LSD passes.  Same order either way */
     RRX_TUNING_TRACE_RAYS_PER_LANE = 8,   /* k sizing a single query's persistent grid (0..64;
-                                             default 2): at most four 256-lane workgroups per CU
-                                             unless 512 x k rays per workgroup need more; below
-                                             that a workgroup per 256 x k rays, at least one per CU
-                                             (single level) or one ray per lane (two level); never
-                                             more than one ray per lane or the resident grid.
-                                             Queries that do not fill the resident grid finish
-                                             sooner on fewer waves per SIMD.  0: the resident grid
-                                             whenever the rays fill it */
+                                             default 2): up to 64 rays for each of 16 waves per CU
+                                             (a scene's: 24), equal shares, as few as one ray a
+                                             wave; above that at most four 256-lane workgroups per
+                                             CU unless 512 x k rays per workgroup need more, at
+                                             least one per 256 x k rays (single level) or one ray
+                                             per lane (two level); never more than one ray per lane
+                                             or the resident grid.  0: the resident grid whenever
+                                             the rays fill it */
     RRX_TUNING_TRACE_2L_MIN_BUSY = 9,     /* RRX_TUNING_TRACE_MIN_BUSY for the two-level kernels
                                              (rrCmdIntersect on a scene, scene requests of
                                              rrxCmdIntersectBatch; 1..64; default 32);

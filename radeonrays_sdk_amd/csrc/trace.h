@@ -35,8 +35,8 @@ constexpr uint32_t kDefaultMinBusy = 24;
 uint32_t MinBusyLanes();
 void SetMinBusyLanes(uint32_t lanes);
 
-// Tuning of the persistent kernel (process-wide): ray indices a wave takes
-// per queue atomic (32, 64 or 128) and LDS ring entries per lane (8, 16 or
+// Tuning of the persistent kernel (process-wide): rays a wave takes at a time
+// (32, 64 or 128; at most half an even share) and LDS ring entries per lane (8, 16 or
 // 32).  Setters reject other values.  Defaults: the sweep's best on the
 // 1M-triangle heightfield with 4M incoherent rays.
 constexpr uint32_t kDefaultFetch = 128;
@@ -62,11 +62,12 @@ uint32_t LdsStackDepth();
 bool SetLdsStackDepth(uint32_t entries);
 
 // Rays per lane k that size a single query's persistent grid (0..64; setter
-// rejects others): at most four workgroups per CU unless 2 x kBlock x k rays
-// per workgroup need more; below that a workgroup per kBlock x k rays, at
-// least one per CU (single level) or one ray per lane (two level); never
-// more than one ray per lane or the resident grid.  0: the resident grid
-// whenever the rays fill it.
+// rejects others).  Up to 64 rays for each of 16 waves per CU (a scene's: 24):
+// equal shares, as few as one ray a wave.  Above that at most four workgroups
+// per CU unless 2 x kBlock x k rays per workgroup need more, at least one per
+// kBlock x k rays (single level) or one ray per lane (two level); never more
+// than one ray per lane or the resident grid.  0: the resident grid whenever
+// the rays fill it.
 constexpr uint32_t kDefaultRaysPerLane = 2;
 uint32_t RaysPerLane();
 bool SetRaysPerLane(uint32_t rays);
