@@ -559,7 +559,7 @@ __device__ __forceinline__ void PoolTraverse(uint2* pool, uint32_t count, const 
             const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(own_nodes >> 32), slot, 64);
             nodes = reinterpret_cast<const BvhNode*>((uint64_t)hi << 32 | lo);
             n_int = (uint32_t)__shfl((int)bvh.n_int, slot, 64);
-            total = 2 * n_int + 1;  // an entry exists only where there is a node
+            total = (uint32_t)__shfl((int)bvh.total, slot, 64);  // the header's count bounds every node, as in the lanes' loop
             const int kinds = __shfl((bvh.boxes ? 1 : 0) | (bvh.any ? 2 : 0), slot, 64);
             boxes = (kinds & 1) != 0;
             any = (kinds & 2) != 0;
