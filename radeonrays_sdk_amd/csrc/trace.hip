@@ -816,8 +816,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
 // level).  The world ray is in LDS already; an entry inside an instance
 // transforms it again, as entering the instance does, so each step costs
 // that and one more dependent load (the instance's BLAS address), against
-// one step per node of a ray's whole chain.  Every BLAS's nodes follow its
-// header.  A scene of 1,000 instances of 2,000-triangle soups built and
+// one step per node of a ray's whole chain.  A scene of 1,000 instances of 2,000-triangle soups built and
 // traced: 262,144 any-hit rays 1.70 -> 1.08 ms, 40,000 closest-hit rays
 // 1.44 -> 0.46 ms.
 constexpr uint32_t kPoolDepthBits = 7;
@@ -906,17 +905,21 @@ __device__ __forceinline__ void PoolTraverse2L(uint2* pool, uint32_t count, cons
         bool hit = false;
         TriHit h;
         if (e.x != kInvalid) {
-            const BvhNode* nodes = top.nodes;
             uint32_t total = top.total, flags = 0;
             r.ox = world[0][w]; r.oy = world[1][w]; r.oz = world[2][w];
             if (inst != kPoolWorld) {
                 const float4* xp = reinterpret_cast<const float4*>(top.xforms + 2 * (size_t)inst);
                 const float4 x0 = LdG4(xp), x1 = LdG4(xp + 1), x2 = LdG4(xp + 2);
                 const uint8_t* blas = reinterpret_cast<const uint8_t*>(LdG(top.blas_table + inst));
-                nodes = reinterpret_cast<const BvhNode*>(blas + sizeof(AccelHeader));
-                total = LdG(&reinterpret_cast<const AccelHeader*>(blas)->node_count);
-                flags = LdG(&reinterpret_cast<const AccelHeader*>(blas)->flags);
-                LoadNode(nodes, e.x, q0, q1, q2, q3);
+                const AccelHeader* bh = reinterpret_cast<const AccelHeader*>(blas);
+                total = LdG(&bh->node_count);
+                flags = LdG(&bh->flags);
+                const uint64_t offset = LdG(&bh->nodes_offset);
+                // The builders put the nodes right behind the header: fetched
+                // together with it, and again only if it says that they lie
+                // further on (so the first read is inside the buffer too).
+                LoadNode(reinterpret_cast<const BvhNode*>(blas + sizeof(AccelHeader)), e.x, q0, q1, q2, q3);
+                if (offset != sizeof(AccelHeader)) LoadNode(reinterpret_cast<const BvhNode*>(blas + offset), e.x, q0, q1, q2, q3);
                 const float wox = r.ox, woy = r.oy, woz = r.oz;
                 const float wdx = world[3][w], wdy = world[4][w], wdz = world[5][w];
                 const float ox = ((x0.x * wox + x0.y * woy) + x0.z * woz) + x0.w;
@@ -927,7 +930,7 @@ __device__ __forceinline__ void PoolTraverse2L(uint2* pool, uint32_t count, cons
                 const float dz = (x2.x * wdx + x2.y * wdy) + x2.z * wdz;
                 SetupRay(r, ox, oy, oz, r.tmin, dx, dy, dz);
             } else {
-                LoadNode(nodes, e.x, q0, q1, q2, q3);
+                LoadNode(top.nodes, e.x, q0, q1, q2, q3);
                 r.ix = world[6][w]; r.iy = world[7][w]; r.iz = world[8][w];
             }
             const uint32_t c0 = __float_as_uint(q0.w), c1 = __float_as_uint(q1.w);

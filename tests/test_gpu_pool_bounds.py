@@ -11,6 +11,8 @@ from tests.gpu_util import say, to_dev
 pytestmark = pytest.mark.gpu
 
 NODE_COUNT = slice(12, 16)  # AccelHeader.node_count
+NODES_OFFSET = slice(16, 24)  # AccelHeader.nodes_offset
+HEADER = 128
 
 
 def _rays(n, seed, lo=0.0, hi=1.0):
@@ -32,3 +34,34 @@ def test_batch_reads_no_node_past_the_header_count(ctx, dev, query, rays):
     accel.buffer[NODE_COUNT].view(torch.int32)[0] = i.shape[0] - 1
     hits = api.decode_hits(ctx.intersect_batch([(accel, r, query, "full")])[0])
     assert (hits["prim_id"] == rr.RR_INVALID).all()
+
+
+@pytest.mark.parametrize("query", ["closest", "any"])
+@pytest.mark.parametrize("rays", [1, 65, 5000])
+def test_scene_finds_geometry_nodes_where_the_header_says(ctx, dev, query, rays):
+    """An instance of a geometry whose nodes lie further behind its header than the builders put them; what is there
+    instead would read as leaves."""
+    say(f"scene of a geometry with moved nodes, {rays} rays, {query}")
+    v, i = scenes.triangle_soup(4000, scenes.rng_for(82))
+    plain = ctx.build_geometry(to_dev(v, dev), to_dev(i, dev))
+    gap = 4096
+    moved = torch.full((plain.buffer.numel() + gap,), 0xFF, dtype=torch.uint8, device=dev)
+    moved[:HEADER] = plain.buffer[:HEADER]
+    moved[HEADER + gap:] = plain.buffer[HEADER:]
+    moved[NODES_OFFSET].view(torch.int64)[0] = HEADER + gap
+    geometries = (plain, api.Accel(moved, "blas", plain.prim_count))
+    n = 20
+    xf = scenes.random_transforms(np.random.default_rng(83), n, trans=1.0)
+    r = to_dev(_rays(rays, 84, -1.5, 1.5), dev)
+    want = ctx.intersect(ctx.build_scene([plain] * n, xf), r, query, "full_t")
+    scene = ctx.build_scene([geometries[k % 2] for k in range(n)], xf)
+    got = ctx.intersect(scene, r, query, "full_t")
+    torch.cuda.synchronize()
+    assert rays < 5000 or len(set(api.decode_hits(want, "full_t")["inst_id"].tolist()) - {rr.RR_INVALID}) == n
+    assert torch.equal(got, want)
+    saved = autotune.current(ctx.lib)
+    try:
+        autotune.set_(ctx.lib, rr.RRX_TUNING_TRACE_PLAIN, 1)
+        assert torch.equal(ctx.intersect(scene, r, query, "full_t"), want)
+    finally:
+        autotune.apply(ctx.lib, saved)
