@@ -300,14 +300,16 @@ __device__ __forceinline__ void InitQueues(uint32_t* counters, uint32_t n) {
 // own, and it takes `piece` more at a time from queue q.
 struct RayQueue {
     uint32_t next, end, q, piece;
-    uint32_t tries;  // queues found empty
-    bool drained;    // no more rays to take
+    uint32_t blocks;  // workgroups whose waves started with a piece
+    uint32_t tries;   // queues found empty
+    bool drained;     // no more rays to take
 };
 
-// The rays at the head of queue q that the waves starting on it have from
-// the beginning, a piece each: its counter counts those behind them.
-__device__ __forceinline__ uint32_t QueueFirst(uint32_t q, uint32_t piece) {
-    return (gridDim.x + kQueues - 1 - q) / kQueues * (kBlock / 64) * piece;
+// The rays at the head of queue q that the waves of `blocks` workgroups
+// starting on it have from the beginning, a piece each (none for 0): its
+// counter counts those behind them.
+__device__ __forceinline__ uint32_t QueueFirst(uint32_t q, uint32_t piece, uint32_t blocks) {
+    return (blocks + kQueues - 1 - q) / kQueues * (kBlock / 64) * piece;
 }
 
 // A wave's first rays.  When the grid's lanes hold every ray, each wave has
@@ -316,12 +318,24 @@ __device__ __forceinline__ uint32_t QueueFirst(uint32_t q, uint32_t piece) {
 // (all waves at once would wait for each other's: 4M rays of a camera above
 // the 1M-triangle terrain 506 -> 491 us, 4M rays towards a 3,000-triangle
 // soup 337 -> 330).
-__device__ __forceinline__ bool StartQueue(RayQueue& s, uint32_t n, uint32_t part, uint32_t fetch) {
+//
+// A grid for equal shares relies on the pool.  Waves that cannot pool keep
+// equal shares of up to kLoneShare rays; beyond that the query is left to the
+// first `lone` workgroups, the grid that it has without equal shares, and its
+// waves take every piece from the queues (and so refill their lanes).
+// Closest hits in a scene of 524,287 instances, rays from outside / inside,
+// equal shares against the queues: 24,500 rays (4 a wave) 1093/1135 against
+// 1879/2324 us, 49,000 (8) 1640/1485 against 2216/2507, 98,000 (16) 2156/1933
+// against 2051/2416, 393,216 (64) 4543/3675 against 2983/3056.  A first piece
+// without an atomic gave them nothing (98,000 rays from inside 2416 -> 2759).
+constexpr uint32_t kLoneShare = 8;
+__device__ __forceinline__ bool StartQueue(RayQueue& s, uint32_t n, uint32_t part, uint32_t fetch, bool pools, uint32_t lone) {
     const uint32_t waves = gridDim.x * (kBlock / 64);
     const uint32_t share = n / waves + (n % waves != 0);
-    const bool fixed = share <= 64;
+    const bool fixed = share <= (pools ? 64u : kLoneShare);
     s.q = blockIdx.x % kQueues;
     s.piece = fixed ? share : fetch;
+    s.blocks = gridDim.x;
     s.tries = 0;
     const uint32_t block = fixed ? XcdContiguousBlock(blockIdx.x, gridDim.x) : blockIdx.x / kQueues;
     const uint32_t first = fixed ? 0 : s.q * part, end = fixed ? n : min((s.q + 1) * part, n);
@@ -329,6 +343,11 @@ __device__ __forceinline__ bool StartQueue(RayQueue& s, uint32_t n, uint32_t par
     s.next = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)min(first + (uint64_t)w * s.piece, (uint64_t)end));
     s.end = s.next + min(s.piece, end - s.next);
     s.drained = fixed && s.next == s.end;
+    if (!pools && !fixed) {
+        s.blocks = 0;
+        s.end = s.next;
+        s.drained = blockIdx.x >= lone;
+    }
     return fixed;
 }
 
@@ -337,7 +356,7 @@ __device__ __forceinline__ void TakeRays(RayQueue& s, uint32_t* counters, uint32
     while (!s.drained) {
         uint32_t b = 0;
         if (__lane_id() == 0) b = atomicAdd(&counters[s.q * kQueueStride], s.piece);
-        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + QueueFirst(s.q, s.piece);
+        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + QueueFirst(s.q, s.piece, s.blocks);
         const uint32_t end = min((s.q + 1) * part, n);
         if (b < end) {
             s.next = b;
@@ -659,7 +678,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
 
     // Wave-uniform queue state.
     RayQueue rq;
-    const bool fixed = StartQueue(rq, n, part, fetch);
+    const bool fixed = StartQueue(rq, n, part, fetch, true, 0);
     bool pooled = false;  // the wave's last rays go on in a pool
 
     // Lane state.
@@ -1006,7 +1025,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
                                                                   const uint32_t* __restrict__ indirect,
                                                                   void* __restrict__ hits,
                                                                   uint32_t* __restrict__ scratch, uint32_t min_busy,
-                                                                  uint32_t fetch, uint32_t init_queues, uint32_t* err) {
+                                                                  uint32_t fetch, uint32_t lone, uint32_t init_queues, uint32_t* err) {
     __shared__ uint32_t s_stack[kBlock / 64][DEPTH][64];
     // Each lane's world ray: origin xyz, direction xyz and reciprocal
     // direction, restored without divisions when the lane leaves an
@@ -1032,7 +1051,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
 
     // Wave-uniform queue state.
     RayQueue rq;
-    const bool fixed = StartQueue(rq, n, part, fetch);
+    const bool pools = top_prims < kPoolWorld;
+    const bool fixed = StartQueue(rq, n, part, fetch, pools, lone);
     bool pooled = false;  // the wave's last rays go on in a pool
 
     // Lane state: the ray of the level being traversed (the world ray waits
@@ -1083,7 +1103,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
             if (rq.drained) break;
             continue;
         }
-        if (rq.drained && top_prims < kPoolWorld && PoolFits(st, node, leaf, rid)) {
+        if (rq.drained && pools && PoolFits(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -1213,7 +1233,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
             }
             if (!rq.drained && (uint32_t)__popcll(__ballot(1)) < min_busy) break;  // refill (nothing left once rq.drained)
             // Drained, but the pool had no room: try again once a lane is done.
-            if (rq.drained && __ballot(1) != entered) break;
+            if (rq.drained && pools && __ballot(1) != entered) break;
         }
     }
     // The wave's last rays.
@@ -1295,7 +1315,7 @@ __device__ __forceinline__ bool NextBatchChunk(const BatchRequest* __restrict__ 
         // Part `part` holds chunks [first + p_lo, first + p_hi).
         const uint32_t p_lo = (uint32_t)((uint64_t)count * part / kQueues);
         const uint32_t p_hi = (uint32_t)((uint64_t)count * (part + 1) / kQueues);
-        const uint32_t waves = QueueFirst(part, 1);
+        const uint32_t waves = QueueFirst(part, 1, gridDim.x);
         uint32_t* counter = counters + part * kQueueStride;
         uint32_t c = 0;
         if (!started) {
@@ -1920,20 +1940,23 @@ uint32_t FetchFor(uint32_t n, uint32_t blocks, bool two) {
 
 template <bool ANY, bool TWO, int OUT, int DEPTH>
 void LaunchPersistentKernel(uint32_t blocks, hipStream_t s, const uint8_t* a, const float4* r, uint32_t n,
-                            const uint32_t* ind, void* hits, uint32_t* sc, uint32_t mb, uint32_t f, uint32_t init) {
+                            const uint32_t* ind, void* hits, uint32_t* sc, uint32_t mb, uint32_t f, uint32_t lone,
+                            uint32_t init) {
     uint32_t* err = DeviceErrorWords();
-    if (TWO) TracePersistent2LKernel<ANY, OUT, DEPTH><<<blocks, kBlock, 0, s>>>(a, r, n, ind, hits, sc, mb, f, init, err);
+    if (TWO) TracePersistent2LKernel<ANY, OUT, DEPTH><<<blocks, kBlock, 0, s>>>(a, r, n, ind, hits, sc, mb, f, lone, init, err);
     else TracePersistentKernel<ANY, OUT, DEPTH><<<blocks, kBlock, 0, s>>>(a, r, n, ind, hits, sc, mb, f, init, err);
 }
 
 template <bool ANY, bool TWO, int DEPTH>
 void LaunchPersistentDepth(OutputKind out, uint32_t blocks, hipStream_t s, const uint8_t* a, const float4* r,
                            uint32_t n, const uint32_t* ind, void* hits, uint32_t* sc, uint32_t init) {
-    const uint32_t mb = TWO ? MinBusyLanes2L() : MinBusyLanes(), f = FetchFor(n, blocks, TWO);
+    // Equal shares take no pieces, unless the scene is too large for a pool.
+    const uint32_t lone = TWO ? std::min(blocks, QueryBlocks(n, true)) : blocks;
+    const uint32_t mb = TWO ? MinBusyLanes2L() : MinBusyLanes(), f = FetchFor(n, lone, TWO);
     switch (out) {
-        case kOutFullHit: LaunchPersistentKernel<ANY, TWO, kOutFullHit, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, init); break;
-        case kOutInstanceId: LaunchPersistentKernel<ANY, TWO, kOutInstanceId, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, init); break;
-        default: LaunchPersistentKernel<ANY, TWO, kOutFullHitT, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, init); break;
+        case kOutFullHit: LaunchPersistentKernel<ANY, TWO, kOutFullHit, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, lone, init); break;
+        case kOutInstanceId: LaunchPersistentKernel<ANY, TWO, kOutInstanceId, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, lone, init); break;
+        default: LaunchPersistentKernel<ANY, TWO, kOutFullHitT, DEPTH>(blocks, s, a, r, n, ind, hits, sc, mb, f, lone, init); break;
     }
 }
 
