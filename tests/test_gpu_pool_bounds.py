@@ -65,3 +65,39 @@ def test_scene_finds_geometry_nodes_where_the_header_says(ctx, dev, query, rays)
         assert torch.equal(ctx.intersect(scene, r, query, "full_t"), want)
     finally:
         autotune.apply(ctx.lib, saved)
+
+
+@pytest.mark.parametrize("which", ["soup", "scene"])
+def test_pool_of_short_stacks_has_room_to_work(ctx, dev, which):
+    """Long rays, 64 for every wave that pools at once: with eight-entry stacks, whose pool was half reserve, they took
+    4.7 times (a geometry) and 5.2 times (a scene) as long as with 16 entries; the stacks alone make no such
+    difference (a factor of 1.2 for queries that do not pool)."""
+    say(f"pool on eight-entry stacks timed, {which}")
+    if which == "soup":
+        v, i = scenes.triangle_soup(65536, scenes.rng_for(85))
+        accel, n, eye = ctx.build_geometry(to_dev(v, dev), to_dev(i, dev), restructure=True), 260000, (0.5, 0.5, -1.5)
+    else:
+        geometries = []
+        for k in range(8):
+            v, i = scenes.triangle_soup(2000, scenes.rng_for(86, k))
+            geometries.append(ctx.build_geometry(to_dev(v, dev), to_dev(i, dev), restructure=True))
+        xf = scenes.random_transforms(np.random.default_rng(87), 1000, trans=12.0)
+        accel, n, eye = ctx.build_scene([geometries[k % 8] for k in range(1000)], xf), 390000, (0.0, 0.0, -36.0)
+    r = to_dev(scenes.camera_rays(500, n // 500, eye), dev)
+    hits, scratch = ctx.empty(n * 16), ctx.trace_scratch(n)
+    saved = autotune.current(ctx.lib)
+    times = {}
+    try:
+        for _ in range(6):
+            for depth in (8, 16):
+                autotune.set_(ctx.lib, rr.RRX_TUNING_TRACE_LDS_STACK, depth)
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                ctx.intersect(accel, r, "closest", "full", hits=hits, scratch=scratch)
+                b.record()
+                torch.cuda.synchronize()
+                times.setdefault(depth, []).append(a.elapsed_time(b))
+    finally:
+        autotune.apply(ctx.lib, saved)
+    short, usual = (sorted(times[d])[2] for d in (8, 16))
+    assert short < 2 * usual, (short, usual)
