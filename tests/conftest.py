@@ -31,3 +31,18 @@ def dev():
     import torch
 
     return torch.device("cuda", 0)
+
+
+@pytest.fixture(autouse=True)
+def _traversal_mode(request):
+    """A GPU test that switches the process to the plain traversal kernels
+    leaves the following tests the kernels it found."""
+    if request.node.get_closest_marker("gpu") is None:
+        yield
+        return
+    from radeonrays_sdk_amd import autotune, rr
+
+    lib = rr.load()
+    before = autotune.get(lib, rr.RRX_TUNING_TRACE_PLAIN)
+    yield
+    autotune.set_(lib, rr.RRX_TUNING_TRACE_PLAIN, before)
