@@ -454,11 +454,12 @@ __device__ __forceinline__ uint32_t WavePrefixSum(uint32_t v) {
     return v;
 }
 
-// Whether what the lanes have left fits into a pool: nothing spilled to
-// scratch, and room to work.  Every lane of the wave calls it.
-template <int DEPTH>
+// Whether what the lanes have left fits into a pool, with room to work:
+// without SPILLED, only what no lane spilled to scratch.  Every lane of the
+// wave calls it.
+template <bool SPILLED, int DEPTH>
 __device__ __forceinline__ bool PoolFits(const LaneStack<DEPTH>& st, uint32_t node, uint32_t leaf, uint32_t rid) {
-    if (__any(rid != kInvalid && st.gbase != 0)) return false;
+    if (!SPILLED && __any(rid != kInvalid && st.gbase != 0)) return false;
     const uint32_t sum = WavePrefixSum(PoolOwn((uint32_t)st.sp, node, leaf, rid));
     return (uint32_t)__builtin_amdgcn_readlane((int)sum, 63) + kPoolReserve <= (uint32_t)kPoolCapacity<DEPTH>;
 }
@@ -472,14 +473,21 @@ __device__ __forceinline__ bool PoolFits(const LaneStack<DEPTH>& st, uint32_t no
 template <int DEPTH>
 constexpr uint32_t kPoolWide = (kPoolCapacity<DEPTH> - kPoolReserve) / 2;
 
+// The single-level kernel pools what its eight-entry stacks spilled: with a
+// tree deeper than they are, some lane nearly always has spilled (1M-triangle
+// terrain, 2M camera rays, closest / any: 585/561 us without, 367/330 with;
+// 300,000 rays from anywhere in the unit cube 187/170 and 99/98).
+template <int DEPTH>
+constexpr bool kPoolSpilled = DEPTH < 16;
+
 // Turns the wave's stacks into the pool, in place: lane 0's entries on top,
 // each lane's in the order of its stack (a short pool: every ray's first
 // entry above everyone's others).  Returns the number of entries.
-template <int DEPTH>
-__device__ __forceinline__ uint32_t PoolFromStacks(uint32_t (*lds)[64], uint32_t sp, uint32_t node, uint32_t leaf,
-                                                   uint32_t rid) {
+template <bool SPILLED, int DEPTH>
+__device__ __forceinline__ uint32_t PoolFromStacks(const LaneStack<DEPTH>& st, uint32_t node, uint32_t leaf, uint32_t rid) {
     const uint32_t lane = __lane_id();
-    const uint32_t entries = rid != kInvalid ? sp : 0u;
+    const uint32_t sp = (uint32_t)st.sp, entries = rid != kInvalid ? sp : 0u;
+    const uint32_t spilled = SPILLED && rid != kInvalid ? (uint32_t)st.gbase : 0u;
     uint32_t sum = WavePrefixSum(PoolOwn(sp, node, leaf, rid));
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
     const bool lead = total < kPoolWide<DEPTH> && rid != kInvalid && (node != kInvalid || leaf != kInvalid);
@@ -488,19 +496,22 @@ __device__ __forceinline__ uint32_t PoolFromStacks(uint32_t (*lds)[64], uint32_t
     const uint32_t rest = total - (uint32_t)__popcll(leads);
     uint32_t row[DEPTH];
 #pragma unroll
-    for (int i = 0; i < DEPTH; ++i) row[i] = lds[i][lane];
+    for (int i = 0; i < DEPTH; ++i) row[i] = st.lds[i][lane];
     WaveLdsFence();
-    uint2* at = reinterpret_cast<uint2*>(lds) + (rest - sum);
+    uint2* pool = reinterpret_cast<uint2*>(st.lds);
+    uint2* at = pool + (rest - sum);
+    for (uint32_t i = 0; i < spilled; ++i) at[i] = make_uint2(LdG(st.slot((int)i)), lane | i << kPoolSlotBits);
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) {
         __builtin_amdgcn_sched_barrier(0);  // one entry's second word at a time in registers
-        if ((uint32_t)i < entries) at[i] = make_uint2(row[i], lane | (uint32_t)i << kPoolSlotBits);
+        const uint32_t e = spilled + (((uint32_t)i - spilled) & (uint32_t)(DEPTH - 1));  // the entry in row i
+        if (e < entries) at[e] = make_uint2(row[i], lane | e << kPoolSlotBits);
     }
     at += entries;
     const uint32_t word = lane | entries << kPoolSlotBits;
     if (rid != kInvalid && node != kInvalid && (leaf != kInvalid || !lead)) *at++ = make_uint2(node, word);
     if (rid != kInvalid && leaf != kInvalid && !lead) *at = make_uint2(leaf, word);
-    if (lead) reinterpret_cast<uint2*>(lds)[total - 1 - RankIn(leads)] = make_uint2(leaf != kInvalid ? leaf : node, word);
+    if (lead) pool[total - 1 - RankIn(leads)] = make_uint2(leaf != kInvalid ? leaf : node, word);
     WaveLdsFence();
     return total;
 }
@@ -727,7 +738,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
             if (rq.drained) break;
             continue;
         }
-        if (rq.drained && PoolFits(st, node, leaf, rid)) {
+        if (rq.drained && PoolFits<kPoolSpilled<DEPTH>>(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -810,7 +821,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     }
     // The wave's last rays.
     if (pooled) {
-        const uint32_t count = PoolFromStacks<DEPTH>(st.lds, (uint32_t)st.sp, node, leaf, rid);
+        const uint32_t count = PoolFromStacks<kPoolSpilled<DEPTH>>(st, node, leaf, rid);
         PoolHits& best = s_best[threadIdx.x / 64];
         best.u[lane] = bU;
         best.v[lane] = bV;
@@ -1112,7 +1123,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
             if (rq.drained) break;
             continue;
         }
-        if (rq.drained && pools && PoolFits(st, node, leaf, rid)) {
+        if (rq.drained && pools && PoolFits<false>(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -1449,7 +1460,7 @@ __global__ __launch_bounds__(kBlock) void TraceBatchKernel(const BatchRequest* _
             if (drained) break;
             continue;
         }
-        if (drained && PoolFits(st, node, leaf, rid)) {
+        if (drained && PoolFits<false>(st, node, leaf, rid)) {
             pooled = true;
             break;
         }
@@ -1525,7 +1536,7 @@ __global__ __launch_bounds__(kBlock) void TraceBatchKernel(const BatchRequest* _
     }
     // The wave's last rays.
     if (pooled) {
-        const uint32_t count = PoolFromStacks<kLdsStackEntries>(st.lds, (uint32_t)st.sp, node, leaf, rid);
+        const uint32_t count = PoolFromStacks<false>(st, node, leaf, rid);
         PoolHits& best = s_best[threadIdx.x / 64];
         best.u[lane] = bu;
         best.v[lane] = bv;
