@@ -74,8 +74,9 @@ RR_API RRError rrxCmdIntersectWithStats(RRContext        context,
 typedef enum RRxTuning
 {
     RRX_TUNING_TRACE_MIN_BUSY = 0,        /* refill a wave once fewer lanes traverse (1..64; default 24) */
-    RRX_TUNING_TRACE_RAYS_PER_FETCH = 1,  /* rays a wave takes at a time (32, 64, 128; default 128; at
-                                             most half an even share, at least 32) */
+    RRX_TUNING_TRACE_RAYS_PER_FETCH = 1,  /* rays a wave takes at a time (32, 64, 128; default 128; cut
+                                             to half an even share, rounded down to 32s, but not
+                                             below 64 while a share is larger) */
     RRX_TUNING_TRACE_LDS_STACK = 2,       /* LDS stack entries per lane (8, 16, 32; default 16) */
     RRX_TUNING_TRACE_PLAIN = 3,           /* 1: one lane per ray for its whole traversal, no
                                              persistent kernels (default 0, or 1 when the

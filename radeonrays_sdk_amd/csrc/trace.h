@@ -36,9 +36,9 @@ uint32_t MinBusyLanes();
 void SetMinBusyLanes(uint32_t lanes);
 
 // Tuning of the persistent kernel (process-wide): rays a wave takes at a time
-// (32, 64 or 128; at most half an even share) and LDS ring entries per lane (8, 16 or
-// 32).  Setters reject other values.  Defaults: the sweep's best on the
-// 1M-triangle heightfield with 4M incoherent rays.
+// (32, 64 or 128; cut to half an even share, see PieceRays) and LDS ring
+// entries per lane (8, 16 or 32).  Setters reject other values.  Defaults: the
+// sweep's best on the 1M-triangle heightfield with 4M incoherent rays.
 constexpr uint32_t kDefaultFetch = 128;
 constexpr uint32_t kDefaultLdsStack = 16;
 uint32_t RaysPerFetch();

@@ -25,6 +25,7 @@
 #include "device_errors.h"
 #include "rr_device.h"
 #include "trace.h"
+#include "trace_grid.h"
 
 #include <algorithm>
 #include <atomic>
@@ -35,7 +36,7 @@ namespace rr {
 
 namespace {
 
-constexpr int kBlock = 256;
+constexpr int kBlock = kTraceBlock;
 
 // Trace scratch: kQueues ray-queue counters, each on its own 128-byte line,
 // then kSpillEntries stack slots per lane.
@@ -1944,18 +1945,8 @@ uint32_t QueryBlocks(uint64_t n, bool two, bool shares = false) {
 uint32_t BatchBlocks() { return ResidentBlocks(reinterpret_cast<const void*>(&TraceBatchKernel), 1); }
 uint32_t Batch2LBlocks() { return ResidentBlocks(reinterpret_cast<const void*>(&TraceBatch2LKernel), 7); }
 
-// Rays per piece for n rays over `blocks` blocks: the level's tuned value, at
-// most half an even share (as a multiple of 32, at least 32), so that waves
-// whose rays end early find more to take (524,288 rays of a camera, closest
-// hit: 65,536-triangle soup 331 -> 235 us, 1M-triangle terrain 253 -> 211).
-// Smaller ones still cost more in atomics than they balance (1M rays in
-// pieces of 64: terrain 292 -> 227 us, but 3,000-triangle soup 158 -> 172,
-// and 4M rays 330 -> 374).
 uint32_t FetchFor(uint32_t n, uint32_t blocks, bool two) {
-    const uint64_t waves = (uint64_t)blocks * (kBlock / 64);
-    const uint64_t per = (n + 2 * waves - 1) / (2 * waves);
-    const uint32_t f = (uint32_t)std::max<uint64_t>(32, (per + 31) / 32 * 32);
-    return std::min(two ? RaysPerFetch2L() : RaysPerFetch(), f);
+    return PieceRays(n, blocks, two ? RaysPerFetch2L() : RaysPerFetch());
 }
 
 template <bool ANY, bool TWO, int OUT, int DEPTH>
