@@ -33,7 +33,9 @@
 namespace rr {
 
 constexpr int kTreeWindow = 512;  // threads of a workgroup: one leaf, or one published subtree, each
-constexpr uint32_t kTreeGroup = 48;  // about ten published subtrees of each fill a workgroup; at most 64 (one wave scans them)
+constexpr uint32_t kTreeGroup = 48;  // about ten published subtrees of each fill a workgroup
+// One wave scans a group's counts and gives the sum in one entry more.
+static_assert(kTreeGroup < 64, "group_first[children] is written by lane `children`");
 // A contiguous run of keys leaves at most this many subtrees unmerged: those
 // on one side have strictly decreasing prefixes with what lies beyond, and
 // there are at most 60 prefix lengths (30 code bits, then the key position's
@@ -109,7 +111,7 @@ struct TreeLds {
     uint64_t slot_nodes[kTreeWindow / 64];       // of each 64 slots: address of node 0 of their tree, less the first key
     uint32_t slot_leaves[kTreeWindow / 64];      // ... and leaves less one
     uint32_t wave_pending[kTreeWindow / 64];
-    uint32_t group_first[64 + 1];
+    uint32_t group_first[64];
     uint32_t go;
 };
 
