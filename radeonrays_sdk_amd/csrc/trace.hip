@@ -1067,7 +1067,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
     const Transform* xforms = reinterpret_cast<const Transform*>(accel + hdr->transforms_offset);
     const uint64_t* blas_table = reinterpret_cast<const uint64_t*>(accel + hdr->blas_table_offset);
     uint32_t* counters = scratch;
-    const uint32_t lane = __lane_id();
     const uint32_t part = (n + kQueues - 1) / kQueues;
 
     // Wave-uniform queue state.
@@ -1269,7 +1268,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(DEPTH <=
             WriteHit<OUT, true>(hits, rid, best_prim != kInvalid, bu, bv, best_inst, best_prim, ANY ? hit_t : best_t, best_t);
     }
 }
-
 
 template <bool ANY, bool TWO_LEVEL, bool STATS>
 void LaunchOut(OutputKind out, dim3 g, hipStream_t s, const uint8_t* accel, const float4* rays, uint32_t count,

@@ -20,9 +20,11 @@
 // accesses), is gone.  Nodes and leaves go to memory whole and in order
 // through LDS.  The few subtrees whose sibling lies outside (about ten per
 // window) are published in key order, and the last workgroup of kTreeGroup
-// windows does the same with those, and so on up: two or three hand-offs
-// between workgroups for any tree.  Boxes are min and max, so the result
-// does not depend on which workgroup merges what.
+// windows does the same with those, and so on up: as many hand-offs between
+// workgroups as the logarithm of the windows to base kTreeGroup, rounded up
+// (none for one window, one for up to 24,576 leaves, two for up to 1.18M,
+// three for up to 56.6M).  Boxes are min and max, so the result does not
+// depend on which workgroup merges what.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -297,9 +299,9 @@ __device__ __forceinline__ bool BuildWindow(BvhNode* nodes, uint32_t n, uint32_t
 }
 
 // Publishes the workgroup's waiting subtrees, in key order (a thread's
-// subtree contains the thread's entry, and a thread has one at most), as run `run`; returns their number.
-// Every thread calls it (it holds barriers); the stores are complete when it
-// returns.
+// subtree contains the thread's entry, and a thread has one at most), as run
+// `run`; returns their number.  Every thread calls it (it holds barriers); the
+// stores are complete when it returns.
 __device__ __forceinline__ uint32_t PublishRun(bool waits, const TreeRun& r, const TreeScratch& ts, uint32_t run,
                                                TreeLds& s) {
     const uint64_t mask = __ballot(waits);
@@ -324,8 +326,9 @@ __device__ __forceinline__ uint32_t PublishRun(bool waits, const TreeRun& r, con
     return total;
 }
 
-// After a window (waits, r: BuildWindow's result): hand-offs up the levels.  Window `window` of `windows` (> 1) of a tree of n leaves; code(k):
-// sorted code k, in global memory.  Every thread of the workgroup calls it.
+// After a window (waits, r: BuildWindow's result): hand-offs up the levels.
+// Window `window` of `windows` (> 1) of a tree of n leaves; code(k): sorted
+// code k, in global memory.  Every thread of the workgroup calls it.
 template <typename Code>
 __device__ __forceinline__ void FinishTree(BvhNode* __restrict__ nodes, uint32_t n, const Code& code, bool waits, TreeRun& r,
                                            const TreeScratch& ts, uint32_t window, uint32_t windows, TreeLds& s) {
