@@ -1347,7 +1347,7 @@ RRError rrxCmdBuildGeometryBatch(RRContext context, RRBuildOperation build_opera
             b.tri_count = m.tri_count;
             b.flags = (restructure && m.tri_count >= 64) ? rr::kAccelFlagRestructured : 0u;
             const uint32_t mesh_chunks = rr::RefitChunks(m.tri_count);
-            b.first_chunk = rr::BatchFirstChunk(chunks, mesh_chunks);
+            b.first_chunk = rr::BatchFirstChunk(chunks, mesh_chunks, update);
             chunks = b.first_chunk + mesh_chunks;
             host[k] = b;
         }

@@ -42,11 +42,14 @@ inline size_t BatchHeadBytes(uint32_t meshes) {
 // Leaves per refit queue entry.
 constexpr uint32_t kRefitChunk = 64;
 inline uint32_t RefitChunks(uint32_t tris) { return (tris + kRefitChunk - 1) / kRefitChunk; }
-// First chunk of a mesh of `chunks` chunks when `before` chunks precede it:
-// meshes do not cross a workgroup of the tree kernel unless they start one.
+// First chunk of a mesh of `chunks` chunks when `before` chunks precede it.
+// A build: meshes do not cross a workgroup of the tree kernel unless they
+// start one.  An update packs them: its refit takes any mix, and the gaps
+// (5 % of the lanes over 8,192 meshes of 64-16,384 triangles) would only be
+// empty lanes, 2534 against 2452 us.
 constexpr uint32_t kBatchChunksPerWindow = 8;
-inline uint32_t BatchFirstChunk(uint32_t before, uint32_t chunks) {
-    return before % kBatchChunksPerWindow + chunks > kBatchChunksPerWindow
+inline uint32_t BatchFirstChunk(uint32_t before, uint32_t chunks, bool update) {
+    return !update && before % kBatchChunksPerWindow + chunks > kBatchChunksPerWindow
                ? (before + kBatchChunksPerWindow - 1) / kBatchChunksPerWindow * kBatchChunksPerWindow
                : before;
 }
