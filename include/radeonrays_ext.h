@@ -104,7 +104,7 @@ typedef enum RRxTuning
     RRX_TUNING_TRACE_RAYS_PER_LANE = 8,   /* k sizing a single query's persistent grid (0..64;
                                              default 2): up to 64 rays for each of 16 waves per CU
                                              (a scene's: 24), equal shares, as few as one ray a
-                                             wave; above that at most four 256-lane workgroups per
+                                             wave, whatever k >= 1; above that at most four 256-lane workgroups per
                                              CU unless 512 x k rays per workgroup need more, at
                                              least one per 256 x k rays (single level) or one ray
                                              per lane (two level); never more than one ray per lane
@@ -118,8 +118,7 @@ typedef enum RRxTuning
     RRX_TUNING_TRACE_2L_RAYS_PER_FETCH = 10, /* RRX_TUNING_TRACE_RAYS_PER_FETCH for the persistent
                                              two-level kernel (32, 64, 128; default 32) */
     RRX_TUNING_TRACE_BATCH_MIN_BUSY = 11  /* RRX_TUNING_TRACE_MIN_BUSY for the geometry requests
-                                             of rrxCmdIntersectBatch (1..64; default 24; batches of
-                                             many small BLASes run faster at 12) */
+                                             of rrxCmdIntersectBatch (1..64; default 24) */
 } RRxTuning;
 
 RR_API RRError rrxSetTuning(RRxTuning key, uint32_t value);

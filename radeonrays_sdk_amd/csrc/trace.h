@@ -53,8 +53,9 @@ bool SetMinBusyLanes2L(uint32_t lanes);
 uint32_t RaysPerFetch2L();
 bool SetRaysPerFetch2L(uint32_t rays);
 // Refill threshold of the batch kernel's geometry requests (64-ray chunks).
-// 24 suits the serving mix (BLASes of 10k-2M triangles); batches of many
-// small BLASes with short rays run faster at 12.
+// 24 suits the serving mix (BLASes of 10k-2M triangles) and, with the pooled
+// tail, batches of many small BLASes too (2M rays over 8,192: 617 us, 649 at
+// 12, 633 at 32).
 constexpr uint32_t kDefaultMinBusyBatch = 24;
 uint32_t MinBusyLanesBatch();
 bool SetMinBusyLanesBatch(uint32_t lanes);
@@ -63,7 +64,9 @@ bool SetLdsStackDepth(uint32_t entries);
 
 // Rays per lane k that size a single query's persistent grid (0..64; setter
 // rejects others).  Up to 64 rays for each of 16 waves per CU (a scene's: 24):
-// equal shares, as few as one ray a wave.  Above that at most four workgroups
+// equal shares, as few as one ray a wave, whatever k >= 1 (with the rule below
+// 1,000 to 262,144 rays took 1.3 to 3.2 times as long on a geometry, k = 64,
+// and 0.96 to 4.7 times on a scene).  Above that at most four workgroups
 // per CU unless 2 x kBlock x k rays per workgroup need more, at least one per
 // kBlock x k rays (single level) or one ray per lane (two level); never more
 // than one ray per lane or the resident grid.  0: the resident grid whenever
