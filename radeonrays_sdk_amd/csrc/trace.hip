@@ -1908,7 +1908,8 @@ uint32_t PersistentBlocks(bool two) {
 // from inside 112 -> 83) as it loses on others (camera 168 -> 188).  A
 // scene's rays are longer: 24 waves per CU (1,000 instances built and
 // 262,144 rays traced: 1074 -> 945 us; 300 instances, 180,000 rays: 148 ->
-// 118).  The grid may have more lanes than rays (SpillStart).
+// 118).  The grid may have more lanes than rays (SpillStart); a scene too large
+// to pool uses it only for shares of a few rays (kLoneShare).
 //
 // Otherwise never more than one ray per lane and never more
 // than four workgroups per CU (four waves per SIMD) unless 512 x k rays per
